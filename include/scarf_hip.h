@@ -246,6 +246,15 @@ int sh_knn_screen(const void *qpack, int64_t nq, const void *rpack, int64_t nr,
                   uint64_t *cand_keys, int32_t *cand_cnt, void *workspace,
                   size_t workspace_bytes, sh_stream_t stream);
 size_t sh_knn_screen_workspace(int64_t nq, int32_t pool, int32_t n_slices);
+/* One candidate pool per query over all references (cand_keys [nq x pool] sorted,
+ * cand_cnt [nq]), the same pool as sh_knn_screen with one slice.  A pass over a sample of
+ * the references first bounds every query's pool-th smallest key; the scan starts from
+ * that bound, so few keys are inserted and the references can be cut into as many slices
+ * as fill the GPU.  sh_knn_rerank takes the result with n_slices = 1. */
+int sh_knn_pool(const void *qpack, int64_t nq, const void *rpack, int64_t nr, int32_t D,
+                int dtype, int32_t pool, uint64_t *cand_keys, int32_t *cand_cnt,
+                void *workspace, size_t workspace_bytes, sh_stream_t stream);
+size_t sh_knn_pool_workspace(int64_t nq, int64_t nr, int32_t D, int dtype, int32_t pool);
 /* Self queries: query q is reference self_idx[q] (self_idx non-NULL) or
  * self_offset + q (self_offset >= 0); k + 1 neighbours are ranked and the query's
  * own column removed as fix_knn_query does.  Neither: a plain k-neighbour query.

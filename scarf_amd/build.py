@@ -47,7 +47,8 @@ COMMON_FLAGS = [
 # keeps them in VGPRs too (128 accumulator AGPRs on top of its VGPRs would leave one wave
 # per SIMD; in VGPRs it runs two)
 EXTRA_FLAGS = {
-    "sh_knn.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form", "-fno-honor-nans"],
+    **{f"sh_knn{t}.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form", "-fno-honor-nans"]
+       for t in ("", "_bf16", "_fp8", "_f32")},
     "sh_gram.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form"],
 }
 

@@ -2,36 +2,16 @@
 // low-precision screen.  Replaces scarf's hnswlib index (ann.py:14-28, 194-205,
 // 290-326) and fix_knn_query (ann.py:31-52).
 //
-// Screen: the MFMA computes s(q, r) = ||r||^2 - 2 q.r directly: reference rows are
-// packed as [r, ||r||^2 (split over 1 or 3 slots), 0...] and query rows as
-// [-2q, 1, ..., 0...], so one K-padded dot product gives the ranking key
-// (||q||^2 is the same for every reference of a query and is left out).
-//   A operand = 32 references, B operand = 32 queries, D = 32 x 32 FP32 tile: lane l
-//   holds query l%32 and 16 references 8*(v/4) + 4*(l/32) + v%4.
-// The K axis is split between the two lane halves: half h supplies elements
-// [h*K/2, (h+1)*K/2) of its row, for both operands, so each lane streams one
-// contiguous half-row (the MFMA pairs A and B by the same (half, element) slot,
-// so any such split gives the same dot product).
-//
-// Selection: per (query, reference slice) a candidate buffer of CAP (key, index)
-// pairs in global memory and a threshold tau = the pool-th best key so far.  A
-// 32 x 32 tile is filtered with a 16-value min tree and one compare per query;
-// only tiles with a hit (rare once tau has settled) take the insertion path.  When
-// a buffer nears CAP the owning wave sorts it (bitonic across the wave) and keeps
-// the best `pool`.  Each wave owns its queries, so no cross-wave synchronisation.
-// Optionally each query block first screens a set of seed reference rows (for self
-// queries in locality order: the block's own rows) and starts tau at their pool-th key.
+// The screen (MFMA tiles, threshold filter, candidate buffers) and the threshold pass are
+// in sh_knn_screen.h; this file packs the operands, merges and re-ranks the candidates.
 #include <float.h>
 
-#include <type_traits>
+#include <algorithm>
+#include <cmath>
 
-#include "sh_common.h"
-#include "sh_wave_sort.h"
+#include "sh_knn_screen.h"
 
 namespace sh {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ uint16_t f2bf(float f) {  // round to nearest even
   uint32_t u = __float_as_uint(f);
@@ -188,480 +168,174 @@ __global__ void __launch_bounds__(kPackRows) k_pack_bf16(const float *__restrict
   for (int e = tid; e < rows * K / 2; e += RB) o32[e] = s32[e];
 }
 
-// ---------------------------------------------------------------------------------
-// Screen kernel.
-struct OpF32 {
-  typedef float Frag;
-  static constexpr int EPL = 1;  // elements per lane per MFMA
-  static constexpr int ESZ = 4;
-  static constexpr bool kScaled = false;
-  static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-};
-struct OpBF16 {
-  typedef bf16x8 Frag;
-  static constexpr int EPL = 8;
-  static constexpr int ESZ = 2;
-  static constexpr bool kScaled = false;
-  static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-};
-// FP8 E4M3 with per-row E8M0 scales (MX-style, one scale per lane's 32-element block):
-// the norms enter through the accumulator, read from each row's 16-byte trailer.
-typedef int intx8 __attribute__((ext_vector_type(8)));
-struct OpFP8 {
-  typedef intx8 Frag;
-  static constexpr int EPL = 32;
-  static constexpr int ESZ = 1;
-  static constexpr bool kScaled = true;
-  static __device__ __forceinline__ floatx16 mma_s(Frag a, Frag b, floatx16 c, int sa, int sb) {
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, sa, 0, sb);
-  }
-  static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
-    return mma_s(a, b, c, 127, 127);
-  }
-};
-
-
-constexpr int kSliceAlign = 128;       // reference slices start on this multiple
-constexpr float kOpen = FLT_MAX;       // threshold of a pool that is not full yet
-
-// QG: 32-query groups per wave; MINB: resident workgroups per CU the kernel is compiled
-// for (its register budget).  Two groups at three workgroups per CU measured faster than
-// four groups at two (BF16 K=64, 1M x 1M: 215 ms against 231 ms) and than one group at
-// four (176 ms against 184 ms).
-template <class Op, int K>
-struct ScreenShape {
-  static constexpr int QG = 2;
-  static constexpr int QPB = 4 * 32 * QG;  // queries per workgroup
-  static constexpr int MINB = 3;
-};
-// Register budget of one instantiation: three workgroups per CU (168 VGPRs) unless the
-// query fragments or the compaction sort need more -- the FP8 screen at K >= 128 and the
-// 1024-key buffers -- which then run two per CU instead of spilling to scratch.  The BF16
-// screen at K <= 64 with 256-key buffers runs four per CU (128 VGPRs; its spills fall
-// outside the tile loop): 166.6 against 174.6 ms at 1M x 1M, alternated runs on one GPU.
-// The FP8 screen at K = 128 with 512-key buffers needs 165 VGPRs with the late index add
-// (append_quad) and so runs three per CU instead of two.
-template <class Op, int K, int CAP>
-constexpr bool screen_late() {
-  return (std::is_same<Op, OpBF16>::value && K <= 64 && CAP <= 256) ||
-         (std::is_same<Op, OpFP8>::value && K > 64 && K <= 128 && CAP == 512);
-}
-template <class Op, int K, int CAP>
-constexpr int screen_minb() {
-  if constexpr (std::is_same<Op, OpBF16>::value && K <= 64 && CAP <= 256) return 4;
-  if constexpr (std::is_same<Op, OpFP8>::value && K > 64 && K <= 128 && CAP == 512) return 3;
-  return (Op::kScaled && K >= 128) || CAP >= 1024 ? 2 : ScreenShape<Op, K>::MINB;
-}
-
-// Candidate buffer of one (query, slice): CAP keys in two halves of CAP / 2, one per lane
-// half (lanes n and n + 32 both serve query n); each lane appends to its own half with a
-// register counter, so inserting needs no atomics.  Compaction (the whole wave, for one
-// query) sorts both halves' c0 + c1 keys, keeps the best `pool` split between the two
-// halves (or writes them to `out`), and returns the new threshold: the pool-th key once
-// the query has seen `pool` candidates, else kOpen.
-template <int CAP>
-__device__ __forceinline__ int compact_pair(uint64_t *base, int c0, int c1, int pool,
-                                            uint64_t *out, int32_t *out_cnt, float &tau_new) {
-  constexpr int E = CAP / 64;
-  constexpr int HALF = CAP / 2;
+// A query's starting threshold from the threshold pass: the rank-th smallest of its `m`
+// slot minima (k_bound), one wave per query.  The orderable images are searched bit by bit
+// from the top (count the values at or below a prefix); the low kTauSkip bits are left set,
+// which only raises the threshold.  Fewer than `rank` finite minima leave it open.
+constexpr int kTauSkip = 4;
+template <int EL>
+__global__ void __launch_bounds__(256) k_tau(const float *__restrict__ slot_min, int64_t nq,
+                                             int m, int rank, float *__restrict__ tau0,
+                                             int32_t *__restrict__ zero) {
   const int lane = threadIdx.x & 63;
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-  uint64_t v[E];
+  if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
+  const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (q >= nq) return;
+  uint32_t v[EL];
 #pragma unroll
-  for (int i = 0; i < E; ++i) {
-    const int e = lane * E + i;
-    v[i] = e < c0 ? base[e] : (e - c0 < c1 ? base[HALF + (e - c0)] : ~0ull);
+  for (int i = 0; i < EL; ++i) {
+    const int e = i * 64 + lane;
+    v[i] = e < m ? float_ord(slot_min[q * m + e]) : 0xffffffffu;
   }
-  wave_bitonic_sort<E>(v);
-  const int total = c0 + c1;
-  const int keep = total < pool ? total : pool;
-  const int k0 = (keep + 1) / 2;
+  uint32_t prefix = 0;
+  for (int bit = 31; bit >= kTauSkip; --bit) {
+    const uint32_t t = prefix | ((1u << bit) - 1u);
+    int below = 0;
 #pragma unroll
-  for (int i = 0; i < E; ++i) {
-    const int e = lane * E + i;
-    if (e < keep) {
-      if (out)
-        out[e] = v[i];
-      else
-        base[e < k0 ? e : HALF + (e - k0)] = v[i];
+    for (int i = 0; i < EL; ++i) below += __popcll(__builtin_amdgcn_ballot_w64(v[i] <= t));
+    if (below < rank) prefix |= 1u << bit;
+  }
+  const uint32_t t = prefix | ((1u << kTauSkip) - 1u);
+  if (lane == 0) {
+    float tau = kOpen;
+    if (t < float_ord(kOpen)) {
+      const float x = ord_float(t);
+      tau = fminf(x + fabsf(x) * 0x1p-16f, kOpen);
     }
-  }
-  const uint64_t kp = wave_elem_u64<E>(v, pool - 1);
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-  if (out_cnt && lane == 0) *out_cnt = keep;
-  tau_new = total >= pool ? ord_float((uint32_t)(kp >> 32)) : kOpen;
-  return keep;
-}
-
-// True when the predicate holds on any lane of the wave (one ballot, no lane shuffles).
-__device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
-
-// Appends this lane's values of one 4-reference quad that pass tau to its buffer half.
-// Queries past the batch end carry tau = -inf, so nothing of theirs passes.
-// LATE: the reference index is added inside the store (an asm statement the compiler
-// cannot hoist).  Hoisted, a tile that takes this path computes all 16 indices and keeps
-// them in registers, which the four-workgroups-per-CU budget cannot spare; at three per CU
-// the hoisted form is faster.
-template <int V, bool LATE>
-__device__ __forceinline__ void append_one(const floatx16 &acc, float tau, uint32_t ref0,
-                                           uint64_t *half, int &cnt) {
-  constexpr int kOff = 8 * (V >> 2) + (V & 3);  // the value's reference within the tile
-  if (acc[V] <= tau) {
-    uint32_t ref;
-    if constexpr (LATE)
-      asm volatile("v_add_u32 %0, %1, %2" : "=v"(ref) : "i"(kOff), "v"(ref0));
-    else
-      ref = ref0 + (uint32_t)kOff;
-    half[cnt] = make_key(acc[V], ref);
-    ++cnt;
+    tau0[q] = tau;
   }
 }
 
-template <int V0, bool LATE>
-__device__ __forceinline__ void append_quad(const floatx16 &acc, float tau, uint32_t ref0,
-                                            uint64_t *half, int &cnt) {
-  append_one<V0, LATE>(acc, tau, ref0, half, cnt);
-  append_one<V0 + 1, LATE>(acc, tau, ref0, half, cnt);
-  append_one<V0 + 2, LATE>(acc, tau, ref0, half, cnt);
-  append_one<V0 + 3, LATE>(acc, tau, ref0, half, cnt);
-}
-
-template <class Op, int K, int CAP>
-__global__ void __launch_bounds__(256, (screen_minb<Op, K, CAP>())) k_screen(
-    const typename Op::Frag *__restrict__ Qp_, int64_t nq, const unsigned char *__restrict__ Rp,
-    int64_t nr, int64_t slice_len, int S, int pool, const int64_t *__restrict__ seeds,
-    uint64_t *__restrict__ buf, uint64_t *__restrict__ out, int32_t *__restrict__ out_cnt) {
-  typedef typename Op::Frag Frag;
-  constexpr int QG = ScreenShape<Op, K>::QG;
-  constexpr bool kLate = screen_late<Op, K, CAP>();  // see append_quad
-  constexpr int QPW = 32 * QG;                // queries per wave
-  constexpr int QPB = ScreenShape<Op, K>::QPB;
-  constexpr int HALFC = CAP / 2;              // keys per buffer half
-  constexpr int HALF = K / 2;                 // elements per lane half
-  constexpr int NS = HALF / Op::EPL;          // MFMA steps per tile
-  constexpr int GROWB = K * Op::ESZ + (Op::kScaled ? 16 : 0);  // packed row bytes in HBM
-  constexpr int ROWB = K * Op::ESZ + 16;      // LDS row bytes (pad or FP8 trailer)
-  constexpr int CHUNKS = GROWB / 16;          // 16-byte chunks per packed row
-  // references per LDS stage: as many as two stage buffers fit in 48 KiB
-  constexpr int RT = (2 * 128 * ROWB <= 49152) ? 128 : (2 * 64 * ROWB <= 49152) ? 64 : 32;
-  // stage buffers are filled by global_load_lds_dwordx4: each wave instruction writes
-  // 64 consecutive 16-byte chunks (1 KiB), so a buffer is a whole number of KiB
-  constexpr int CPR = ROWB / 16;                      // chunks per padded LDS row
-  constexpr int NINSTR = (RT * CPR + 63) / 64;        // wave instructions per stage
-  constexpr int BUFB = NINSTR * 1024;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds_r[2][BUFB];
-
-  const unsigned char *Qp = reinterpret_cast<const unsigned char *>(Qp_);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, n = lane & 31;
-  const int slice = blockIdx.y;
-  const int64_t r_begin = (int64_t)slice * slice_len;
-  const int64_t r_end = min(nr, r_begin + slice_len);
-  const int qw0 = w * QPW;  // wave's first local query
-  const int64_t qb0 = (int64_t)blockIdx.x * QPB;
-
-  Frag bq[QG][NS];
-  float tau[QG];
-  bool qvalid[QG];
-  int qscale[QG];
-  int cnt[QG];
+// Best `pool` keys of each query over the segments that a sliced scan left in its buffers
+// (two halves per slice, counts in seg_cnt), sorted.  One wave per query.  The counts are
+// scanned into offsets in LDS and every lane finds its keys' segments by bisection, so the
+// loads are independent whatever the counts.  64 * E keys are taken at a time (the usual
+// query has fewer): the pool-th smallest is searched bit by bit on the keys' distance half
+// (count what lies at or below a prefix; on the index half too where distances tie), the
+// keys up to it are packed together in LDS, and only they are sorted: at a million queries
+// of about 240 keys, half the time of sorting them all.
+//
+// BITS: the segments hold plain float bits above the index (k_collect), not make_key's word.
+// fail (or NULL): queries whose keys are incomplete -- a segment that overflowed, or fewer
+// than `need` keys -- are listed there instead, to be screened again.
+// list (or NULL): positions list_base.. of a list of queries whose length the device knows.
+template <int PE, int E, bool BITS>
+__global__ void __launch_bounds__(256) k_pool_merge(
+    const uint64_t *__restrict__ buf, const int32_t *__restrict__ seg_cnt, int64_t n, int S,
+    int cap, int pool, int need, const int32_t *__restrict__ list,
+    const int32_t *__restrict__ list_n, int32_t list_base, int32_t *__restrict__ fail,
+    int32_t *__restrict__ fail_n, int32_t fail_base, uint64_t *__restrict__ out,
+    int32_t *__restrict__ out_cnt) {
+  extern __shared__ uint64_t merge_lds[];  // [4][pool] keys, then [4][2 S] offsets
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t p = (int64_t)blockIdx.x * 4 + w;
+  if (list) n = min(n, (int64_t)*list_n - list_base);
+  if (p >= n) return;
+  const int ns = 2 * S, room = cap / 2;
+  uint64_t *kept = merge_lds + w * pool;
+  int *off = reinterpret_cast<int *>(merge_lds + 4 * pool) + w * ns;
+  int total = 0;
+  bool over = false;
+  for (int b = 0; b < ns; b += 64) {
+    const int c = b + lane < ns ? seg_cnt[p * ns + b + lane] : 0;
+    over |= c > room;
+    int inc = c;
 #pragma unroll
-  for (int g = 0; g < QG; ++g) {
-    const int64_t q = qb0 + qw0 + g * 32 + n;
-    qvalid[g] = q < nq;
-    tau[g] = qvalid[g] ? kOpen : -INFINITY;  // a query past the batch end never passes
-    cnt[g] = 0;
-    qscale[g] = 127;
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-      bq[g][s] = qvalid[g] ? *reinterpret_cast<const Frag *>(
-                                 Qp + q * GROWB + (h * HALF + s * Op::EPL) * Op::ESZ)
-                           : Frag{};
-    if (Op::kScaled && qvalid[g])
-      qscale[g] = *reinterpret_cast<const int32_t *>(Qp + q * GROWB + K * Op::ESZ + 4);
-  }
-
-  // double buffering: stage t+1 streams into the other buffer (LDS DMA) while stage t
-  // computes.  Chunk ci of a stage lands at byte 16*ci: row ci / CPR, column chunk
-  // ci % CPR; the padding chunk of each row and rows past the slice re-read a valid
-  // address (their values are never used).
-  // Byte offset of this lane's chunk within a stage for each of its wave's instructions
-  // (instruction j = w + 4 i fills LDS bytes [1024 j, 1024 j + 1024)); the padding chunk
-  // of a row re-reads the row's first chunk (its value is never used).
-  constexpr int JPW = (NINSTR + 3) / 4;  // instructions per wave per stage (at most)
-  // rows the chunk layout touches per stage (can exceed RT by one when RT * CPR is not a
-  // multiple of 64)
-  constexpr int RROWS = (64 * NINSTR + CPR - 1) / CPR;
-  uint32_t choff[JPW];
-  int chrow[JPW];
-#pragma unroll
-  for (int i = 0; i < JPW; ++i) {
-    const int ci = 64 * (w + 4 * i) + lane;
-    const int rr = ci / CPR, c = ci % CPR;
-    chrow[i] = rr;
-    choff[i] = (uint32_t)(rr * GROWB + (c < CHUNKS ? c : 0) * 16);
-  }
-#define SH_SCREEN_FETCH(T0, B)                                                           \
-  {                                                                                      \
-    const unsigned char *stage = Rp + (T0) * GROWB;                                     \
-    const bool whole = (T0) + RROWS <= r_end; /* uniform: no row past the slice */       \
-    _Pragma("unroll") for (int i = 0; i < JPW; ++i) {                                    \
-      const int j = w + 4 * i;                                                           \
-      if (j < NINSTR) {                                                                  \
-        const unsigned char *src;                                                        \
-        if (whole) {                                                                     \
-          src = stage + choff[i];                                                        \
-        } else { /* rows past the slice re-read its last row */                          \
-          const int64_t last = r_end - 1 - (T0);                                         \
-          const int64_t over = chrow[i] > last ? (int64_t)chrow[i] - last : 0;           \
-          src = stage + choff[i] - over * GROWB;                                         \
-        }                                                                                \
-        __builtin_amdgcn_global_load_lds(                                                \
-            (const void *)src,                                                           \
-            (__attribute__((address_space(3))) void *)(&lds_r[(B)][1024 * j]), 16, 0, 0); \
-      }                                                                                  \
-    }                                                                                    \
-  }
-
-  // Seeding: before the scan, every query of the workgroup screens the workgroup's QPB
-  // seed references (seeds[qb0 .. qb0 + QPB), distinct rows of the reference set, e.g.
-  // the block's own rows when queries are the references in locality order) and starts
-  // from the pool-th smallest of those keys instead of an open threshold.  The seeds are
-  // references of the slice, screened by the same MFMA arithmetic, so at least `pool`
-  // references have a key at or below that threshold and the kept pool is the same; the
-  // scan only skips candidates that could not have stayed.  (A 2^-16 relative margin
-  // keeps this true even if a key were rounded differently in another tile position.)
-  static_assert(QPB % 64 == 0 && QPB <= 256, "at most one seed slot per thread");
-  static_assert(QPB % RT == 0 && (QPB / 32) * 16 <= HALFC, "seed stages must fit the buffer");
-  if (seeds != nullptr && r_begin < r_end) {
-    __shared__ uint32_t seed_row[QPB];
-    __shared__ uint32_t seed_bad[QPB / 32];  // bit s of word i: slot 32 i + s has no seed
-    if (threadIdx.x < QPB) {  // whole waves
-      const int64_t q = qb0 + threadIdx.x;
-      const int64_t r = q < nq ? seeds[q] : -1;
-      const bool ok = r >= r_begin && r < r_end;
-      seed_row[threadIdx.x] = (uint32_t)(ok ? r : r_begin);
-      const uint64_t bad = __ballot(!ok);
-      if (lane == 0) {
-        seed_bad[2 * w] = (uint32_t)bad;
-        seed_bad[2 * w + 1] = (uint32_t)(bad >> 32);
-      }
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(inc, o, kWave);
+      if (lane >= o) inc += up;
     }
-    __syncthreads();
-    for (int s0 = 0; s0 < QPB; s0 += RT) {
-      // gather the stage's seed rows: LDS row rr holds seed slot s0 + rr (rows the chunk
-      // layout touches past the stage re-read a valid row; they are never used)
-#pragma unroll
-      for (int i = 0; i < JPW; ++i) {
-        const int j = w + 4 * i;
-        if (j < NINSTR) {
-          const int slot = s0 + chrow[i];
-          const uint32_t row = seed_row[slot < QPB ? slot : 0];
-          const unsigned char *src =
-              Rp + (int64_t)row * GROWB + (choff[i] - (uint32_t)(chrow[i] * GROWB));
-          __builtin_amdgcn_global_load_lds(
-              (const void *)src, (__attribute__((address_space(3))) void *)(&lds_r[0][1024 * j]),
-              16, 0, 0);
-        }
-      }
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-#pragma unroll
-      for (int sub = 0; sub < RT / 32; ++sub) {
-        floatx16 acc[QG];
-        if constexpr (Op::kScaled) {
-          floatx16 nrm;
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            nrm[v] = *reinterpret_cast<const float *>(
-                &lds_r[0][(sub * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * ROWB + K * Op::ESZ]);
-#pragma unroll
-          for (int g = 0; g < QG; ++g) acc[g] = nrm;
-        } else {
-#pragma unroll
-          for (int g = 0; g < QG; ++g)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[g][v] = 0.f;
-        }
-        const unsigned char *arow = &lds_r[0][(sub * 32 + n) * ROWB + h * HALF * Op::ESZ];
-        int ascale = 127;
-        if constexpr (Op::kScaled)
-          ascale = *reinterpret_cast<const int32_t *>(
-              &lds_r[0][(sub * 32 + n) * ROWB + K * Op::ESZ + 4]);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          Frag a = *reinterpret_cast<const Frag *>(arow + s * Op::EPL * Op::ESZ);
-#pragma unroll
-          for (int g = 0; g < QG; ++g) {
-            if constexpr (Op::kScaled)
-              acc[g] = Op::mma_s(a, bq[g][s], acc[g], ascale, qscale[g]);
-            else
-              acc[g] = Op::mma(a, bq[g][s], acc[g]);
-          }
-        }
-        const uint32_t badw = seed_bad[(s0 >> 5) + sub];
-#pragma unroll
-        for (int g = 0; g < QG; ++g) {
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if ((badw >> (8 * (v >> 2) + 4 * h + (v & 3))) & 1u) acc[g][v] = INFINITY;
-          const int64_t q = qb0 + qw0 + g * 32 + n;
-          uint64_t *half = buf + ((qvalid[g] ? q : 0) * S + slice) * CAP + h * HALFC;
-          append_quad<0, kLate>(acc[g], tau[g], 0u, half, cnt[g]);
-          append_quad<4, kLate>(acc[g], tau[g], 0u, half, cnt[g]);
-          append_quad<8, kLate>(acc[g], tau[g], 0u, half, cnt[g]);
-          append_quad<12, kLate>(acc[g], tau[g], 0u, half, cnt[g]);
-        }
-      }
-      __syncthreads();  // the next stage overwrites the buffer
-    }
-    // each query's threshold: the pool-th smallest seed key (open below `pool` seeds);
-    // the seed keys themselves are dropped, the scan meets those references again
-#pragma unroll
-    for (int g = 0; g < QG; ++g) {
-      for (int src = 0; src < 32; ++src) {
-        const int64_t q = qb0 + qw0 + g * 32 + src;
-        if (q >= nq) break;
-        const int c0 = __builtin_amdgcn_readlane(cnt[g], src);
-        const int c1 = __builtin_amdgcn_readlane(cnt[g], src + 32);
-        float tnew;
-        compact_pair<CAP>(buf + (q * S + slice) * CAP, c0, c1, pool, nullptr, nullptr, tnew);
-        if (n == src)
-          tau[g] = tnew < kOpen ? fminf(tnew + fabsf(tnew) * 0x1p-16f, kOpen) : kOpen;
-      }
-      cnt[g] = 0;
-    }
+    if (b + lane < ns) off[b + lane] = total + inc - c;
+    total += __shfl(inc, 63, kWave);
   }
-
-  int b = 0;
-  if (r_begin < r_end) {
-    SH_SCREEN_FETCH(r_begin, 0)
+  if (fail && (wave_any(over) || total < need)) {
+    if (lane == 0) fail[atomicAdd(fail_n, 1)] = fail_base + (int32_t)p;
+    return;
   }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  for (int64_t t0 = r_begin; t0 < r_end; t0 += RT) {
-    const int64_t tn = t0 + RT;
-    if (tn < r_end) {
-      SH_SCREEN_FETCH(tn, b ^ 1)
-    }
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  int have = 0, next = 0;  // keys kept in LDS, keys taken in
+  do {
+    uint64_t v[E];
+    const int fresh = min(total - next, 64 * E - have);
+    const int m = have + fresh;
 #pragma unroll
-    for (int sub = 0; sub < RT / 32; ++sub) {
-      const int64_t rb = t0 + sub * 32;
-      if (rb >= r_end) continue;
-      floatx16 acc[QG];
-      if constexpr (Op::kScaled) {
-        // accumulator starts at ||r||^2 of each of the lane's 16 references
-        floatx16 nrm;
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-          nrm[v] = *reinterpret_cast<const float *>(
-              &lds_r[b][(sub * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * ROWB + K * Op::ESZ]);
-#pragma unroll
-        for (int g = 0; g < QG; ++g) acc[g] = nrm;
-      } else {
-#pragma unroll
-        for (int g = 0; g < QG; ++g)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) acc[g][v] = 0.f;
-      }
-      const unsigned char *arow = &lds_r[b][(sub * 32 + n) * ROWB + h * HALF * Op::ESZ];
-      // LLVM's small-GEMM interleave of the fragment LDS reads with the MFMAs: 175.1 ->
-      // 172.3 ms for the 1M BF16 screen, alternated runs on one GPU
-      __builtin_amdgcn_iglp_opt(0);
-      int ascale = 127;
-      if constexpr (Op::kScaled)
-        ascale = *reinterpret_cast<const int32_t *>(&lds_r[b][(sub * 32 + n) * ROWB + K * Op::ESZ + 4]);
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        Frag a = *reinterpret_cast<const Frag *>(arow + s * Op::EPL * Op::ESZ);
-#pragma unroll
-        for (int g = 0; g < QG; ++g) {
-          if constexpr (Op::kScaled)
-            acc[g] = Op::mma_s(a, bq[g][s], acc[g], ascale, qscale[g]);
+    for (int i = 0; i < E; ++i) {
+      const int e = i * 64 + lane;
+      v[i] = ~0ull;
+      if (e < have) {
+        v[i] = kept[e];
+      } else if (e < m) {
+        const int src = next + (e - have);
+        int lo = 0, hi = ns - 1;  // last segment whose offset is <= src
+        while (lo < hi) {
+          const int mid = (lo + hi + 1) >> 1;
+          if (off[mid] <= src)
+            lo = mid;
           else
-            acc[g] = Op::mma(a, bq[g][s], acc[g]);
+            hi = mid - 1;
         }
-      }
-      if (rb + 32 > r_end) {  // references past the slice end never pass
-#pragma unroll
-        for (int g = 0; g < QG; ++g)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int64_t ref = rb + 8 * (v >> 2) + 4 * h + (v & 3);
-            if (ref >= r_end) acc[g][v] = INFINITY;
-          }
-      }
-      // quad minima, then the tile minimum, per query group
-      float m4[QG][4];
-      bool hit[QG];
-      bool any_hit = false;
-#pragma unroll
-      for (int g = 0; g < QG; ++g) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          m4[g][j] = fminf(fminf(acc[g][4 * j], acc[g][4 * j + 1]),
-                           fminf(acc[g][4 * j + 2], acc[g][4 * j + 3]));
-        const float m = fminf(fminf(m4[g][0], m4[g][1]), fminf(m4[g][2], m4[g][3]));
-        hit[g] = m <= tau[g];
-        any_hit |= hit[g];
-      }
-      if (wave_any(any_hit)) {
-        // lane's first reference of the tile (quads add 8 * (v / 4) + v % 4)
-        const uint32_t ref0 = (uint32_t)(rb + 4 * h);
-#pragma unroll
-        for (int g = 0; g < QG; ++g) {
-          if (!wave_any(hit[g])) continue;
-          const int64_t q = qb0 + qw0 + g * 32 + n;
-          uint64_t *half = buf + ((qvalid[g] ? q : 0) * S + slice) * CAP + h * HALFC;
-          if (wave_any(m4[g][0] <= tau[g]))
-            append_quad<0, kLate>(acc[g], tau[g], ref0, half, cnt[g]);
-          if (wave_any(m4[g][1] <= tau[g]))
-            append_quad<4, kLate>(acc[g], tau[g], ref0, half, cnt[g]);
-          if (wave_any(m4[g][2] <= tau[g]))
-            append_quad<8, kLate>(acc[g], tau[g], ref0, half, cnt[g]);
-          if (wave_any(m4[g][3] <= tau[g]))
-            append_quad<12, kLate>(acc[g], tau[g], ref0, half, cnt[g]);
-          // compact every query of the group one of whose halves cannot take a tile
-          const uint64_t mk = __ballot(cnt[g] > HALFC - 16);
-          uint32_t mq = (uint32_t)(mk | (mk >> 32));
-          while (mq) {
-            const int src = __ffs(mq) - 1;
-            mq &= mq - 1;
-            const int c0 = __builtin_amdgcn_readlane(cnt[g], src);
-            const int c1 = __builtin_amdgcn_readlane(cnt[g], src + 32);
-            const int64_t qs = qb0 + qw0 + g * 32 + src;
-            float tnew;
-            const int keep = compact_pair<CAP>(buf + (qs * S + slice) * CAP, c0, c1, pool,
-                                               nullptr, nullptr, tnew);
-            if (n == src) {
-              cnt[g] = h == 0 ? (keep + 1) / 2 : keep - (keep + 1) / 2;
-              tau[g] = tnew;
-            }
-          }
-        }
+        v[i] = buf[(p * S + (lo >> 1)) * cap + (lo & 1) * room + (src - off[lo])];
+        if (BITS) v[i] = make_key(__uint_as_float((uint32_t)(v[i] >> 32)), (uint32_t)v[i]);
       }
     }
-    __builtin_amdgcn_s_waitcnt(0);  // the next stage's DMA has landed
-    __syncthreads();
-    b ^= 1;
-  }
-#undef SH_SCREEN_FETCH
-  // final: sort each query's buffer and emit its best `pool`
+    next += fresh;
+    uint32_t t_hi = 0xffffffffu, t_lo = 0xffffffffu;  // the last key to keep
+    if (m > pool) {
+      uint32_t prefix = 0;
+      for (int bit = 31; bit >= 0; --bit) {
+        const uint32_t t = prefix | ((1u << bit) - 1u);
+        int c = 0;
 #pragma unroll
-  for (int g = 0; g < QG; ++g) {
-    for (int src = 0; src < 32; ++src) {
-      const int64_t q = qb0 + qw0 + g * 32 + src;
-      if (q >= nq) break;
-      const int c0 = __builtin_amdgcn_readlane(cnt[g], src);
-      const int c1 = __builtin_amdgcn_readlane(cnt[g], src + 32);
-      float tnew;
-      compact_pair<CAP>(buf + (q * S + slice) * CAP, c0, c1, pool, out + (q * S + slice) * pool,
-                        out_cnt + q * S + slice, tnew);
+        for (int i = 0; i < E; ++i)
+          if (64 * i < m) c += __popcll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) <= t));
+        if (c < pool) prefix |= 1u << bit;
+      }
+      t_hi = prefix;
+      int below = 0, upto = 0;
+#pragma unroll
+      for (int i = 0; i < E; ++i)
+        if (64 * i < m) {
+          below += __popcll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) < t_hi));
+          upto += __popcll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) <= t_hi));
+        }
+      if (upto > pool) {  // equal distances at the cut: the lower indices stay
+        prefix = 0;
+        for (int bit = 31; bit >= 0; --bit) {
+          const uint32_t t = prefix | ((1u << bit) - 1u);
+          int c = below;
+#pragma unroll
+          for (int i = 0; i < E; ++i)
+            if (64 * i < m)
+              c += __popcll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) == t_hi &&
+                                                        (uint32_t)v[i] <= t));
+          if (c < pool) prefix |= 1u << bit;
+        }
+        t_lo = prefix;
+      }
     }
-  }
+    const uint64_t last = ((uint64_t)t_hi << 32) | t_lo;
+    have = 0;
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+      if (64 * i < m) {
+        const bool keep = i * 64 + lane < m && v[i] <= last;
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(keep);
+        if (keep) kept[have + __popcll(mask & ((1ull << lane) - 1ull))] = v[i];
+        have += __popcll(mask);
+      }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } while (next < total);
+  uint64_t s[PE];
+#pragma unroll
+  for (int i = 0; i < PE; ++i) s[i] = lane * PE + i < have ? kept[lane * PE + i] : ~0ull;
+  wave_bitonic_sort<PE>(s);
+  const int64_t q = list ? list[list_base + p] : p;
+#pragma unroll
+  for (int i = 0; i < PE; ++i)
+    if (lane * PE + i < have) out[q * pool + lane * PE + i] = s[i];
+  if (lane == 0) out_cnt[q] = have;
 }
 
 // Exact FP64 squared distance, terms added in feature order, no contraction: the
@@ -1061,14 +735,12 @@ extern "C" size_t sh_knn_screen_workspace(int64_t nq, int32_t pool, int32_t n_sl
   return (size_t)nq * n_slices * screen_cap(pool) * sizeof(uint64_t);
 }
 
-template <class Op, int K, int CAP>
-static void launch_screen(hipStream_t st, const void *qpack, int64_t nq,
-                          const void *rpack, int64_t nr, int64_t slice_len, int S, int pool,
-                          const int64_t *seeds, uint64_t *buf, uint64_t *out, int32_t *cnt) {
-  dim3 grid((uint32_t)cdiv(nq, ScreenShape<Op, K>::QPB), S);
-  hipLaunchKernelGGL((k_screen<Op, K, CAP>), grid, dim3(256), 0, st,
-                     (const typename Op::Frag *)qpack, nq, (const unsigned char *)rpack, nr,
-                     slice_len, S, pool, seeds, buf, out, cnt);
+// The operand type's launchers (all NULL for an unknown type).
+static KnnOps knn_ops(int dtype) {
+  return dtype == SH_BF16  ? knn_ops_bf16()
+         : dtype == SH_FP8 ? knn_ops_fp8()
+         : dtype == SH_F32 ? knn_ops_f32()
+                           : KnnOps{};
 }
 
 extern "C" int sh_knn_screen(const void *qpack, int64_t nq, const void *rpack, int64_t nr,
@@ -1098,65 +770,318 @@ extern "C" int sh_knn_screen(const void *qpack, int64_t nq, const void *rpack, i
   SH_ARG(S == n_slices, "sh_knn_screen: %d slices requested but %lld references give %d; use "
          "a slice count whose slices hold >= 128 references", n_slices, (long long)nr, S);
   SH_ARG(cdiv(nq, 128) <= 0x7fffffffll, "sh_knn_screen: too many queries");
-  hipStream_t st = (hipStream_t)stream;
-  uint64_t *buf = (uint64_t *)workspace;
-  const bool big = pool > 64;
-  const bool huge = pool > 128;
-#define SH_SCREEN_CASE_1024(OP, KV)                                                          \
-  if (K == KV && huge) {                                                                     \
-    launch_screen<OP, KV, 1024>(st, qpack, nq, rpack, nr, slice_len, S, pool, seed_refs,     \
-                                buf, cand_keys, cand_cnt);                                   \
-    SH_LAUNCH_CHECK("k_screen");                                                             \
-    return SH_OK;                                                                            \
+  const KnnOps ops = knn_ops(dtype);
+  ScreenArgs a = {};
+  a.q = qpack, a.nq = nq, a.r = rpack, a.nr = nr, a.slice_len = slice_len;
+  a.S = S, a.pool = pool, a.seeds = seed_refs;
+  a.buf = (uint64_t *)workspace, a.out = cand_keys, a.out_cnt = cand_cnt;
+  if (ops.screen && ops.screen(K, screen_cap(pool), a, (hipStream_t)stream)) {
+    SH_LAUNCH_CHECK("k_screen");
+    return SH_OK;
   }
-#define SH_SCREEN_CASE(OP, KV)                                                               \
-  if (K == KV) {                                                                             \
-    if (big)                                                                                 \
-      launch_screen<OP, KV, 512>(st, qpack, nq, rpack, nr, slice_len, S, pool, seed_refs,    \
-                                 buf, cand_keys, cand_cnt);                                  \
-    else                                                                                     \
-      launch_screen<OP, KV, 256>(st, qpack, nq, rpack, nr, slice_len, S, pool, seed_refs,    \
-                                 buf, cand_keys, cand_cnt);                                  \
-    SH_LAUNCH_CHECK("k_screen");                                                             \
-    return SH_OK;                                                                            \
-  }
-  if (dtype == SH_BF16) {
-    SH_SCREEN_CASE(OpBF16, 16)
-    SH_SCREEN_CASE(OpBF16, 32)
-    SH_SCREEN_CASE(OpBF16, 48)
-    SH_SCREEN_CASE(OpBF16, 64)
-    SH_SCREEN_CASE(OpBF16, 80)
-    SH_SCREEN_CASE(OpBF16, 96)
-    SH_SCREEN_CASE(OpBF16, 112)
-    SH_SCREEN_CASE(OpBF16, 128)
-  } else if (dtype == SH_FP8) {
-    SH_SCREEN_CASE_1024(OpFP8, 64)
-    SH_SCREEN_CASE_1024(OpFP8, 128)
-    SH_SCREEN_CASE(OpFP8, 64)
-    SH_SCREEN_CASE(OpFP8, 128)
-  } else if (dtype == SH_F32) {
-    SH_SCREEN_CASE(OpF32, 8)
-    SH_SCREEN_CASE(OpF32, 16)
-    SH_SCREEN_CASE(OpF32, 24)
-    SH_SCREEN_CASE(OpF32, 32)
-    SH_SCREEN_CASE(OpF32, 40)
-    SH_SCREEN_CASE(OpF32, 48)
-    SH_SCREEN_CASE(OpF32, 56)
-    SH_SCREEN_CASE(OpF32, 64)
-    SH_SCREEN_CASE(OpF32, 72)
-    SH_SCREEN_CASE(OpF32, 80)
-    SH_SCREEN_CASE(OpF32, 88)
-    SH_SCREEN_CASE(OpF32, 96)
-    SH_SCREEN_CASE(OpF32, 104)
-    SH_SCREEN_CASE(OpF32, 112)
-    SH_SCREEN_CASE(OpF32, 120)
-    SH_SCREEN_CASE(OpF32, 128)
-    SH_SCREEN_CASE(OpF32, 136)
-  }
-#undef SH_SCREEN_CASE
-#undef SH_SCREEN_CASE_1024
   set_error("sh_knn_screen: dtype %d with packed K=%d not supported", dtype, K);
   return SH_EUNSUPPORTED;
+}
+
+// How sh_knn_pool cuts its work.
+namespace sh {
+struct PoolPlan {
+  bool bounded;       // false: too few references for a threshold pass to pay
+  bool collect;       // k_collect (and a second screen of what it lists), else k_screen
+  int shift, rank;    // threshold pass: one sampled row of each 2^shift, rank of the minimum
+  int64_t m;          // sampled rows
+  int S1, per, slots; // slices, minima per lane half, slots per query
+  int64_t len1;
+  int64_t batch1;     // queries per threshold launch (bounds the slot workspace)
+  int S3, cap;        // scan: slices, buffer keys per query and slice
+  int64_t len3;
+  int64_t batch3;     // queries per scan launch (bounds the candidate buffers)
+  size_t off_slots, off_buf, off_cnt, off_fail, bytes;
+};
+constexpr int kCUs = 256;
+constexpr size_t kSlotBytes = (size_t)1 << 30;
+constexpr size_t kBufBytes = (size_t)4 << 30;
+// Second screen: the first kAgain listed queries in kAgainSlices reference slices (a few
+// failed queries must not wait for one workgroup's walk over all references), the rest
+// kAgainBatch at a time in one slice.
+constexpr int64_t kAgain = 4096;
+constexpr int kAgainSlices = 16;
+constexpr int64_t kAgainBatch = 1 << 18;
+
+// Slices that fill `resident` workgroups: the first count from `lo` on whose last wave of
+// workgroups leaves under 7% of the GPU idle, else the best one seen.
+static int pick_slices(int64_t qblocks, int64_t resident, int lo, int hi) {
+  int best = lo;
+  double best_use = 0.0;
+  for (int s = lo; s <= hi; ++s) {
+    const int64_t wgs = qblocks * s;
+    const double use = (double)wgs / (double)(cdiv(wgs, resident) * resident);
+    if (use > best_use + 1e-9) {
+      best_use = use;
+      best = s;
+    }
+    if (best_use >= 0.93) break;
+  }
+  return best;
+}
+
+// Rank of the sampled minimum that becomes the threshold: of a pool the sample holds
+// mean = pool / 2^shift on average (binomial, near Poisson), and exceeds
+// mean + 4.75 sqrt(mean) + 5 with a chance of 1e-7 to 4e-7 for means from 1 to 64.
+static int tau_rank(int pool, int shift) {
+  const double mean = (double)pool / (1 << shift);
+  return shift == 0 ? pool
+                    : std::min(pool, (int)std::ceil(mean + 4.75 * std::sqrt(mean) + 5.0));
+}
+
+static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
+  PoolPlan p = {};
+  const KnnOps ops = knn_ops(dtype);
+  const int64_t qb = std::max<int64_t>(1, cdiv(nq, 256));
+  p.bounded = nr >= 8 * (int64_t)pool;
+  // below about a billion pairs (some 0.1 ms of scan) the launches of the second screen
+  // cost more than k_collect saves over k_screen
+  p.collect = p.bounded && (double)nq * (double)nr >= 1e9;
+  p.cap = screen_cap(pool);
+  p.S1 = p.S3 = 1;
+  p.len3 = align_up((size_t)nr, kSliceAlign);
+  if (p.bounded) {
+    // A sample of 1 / s of the rows costs nr * c_pair / s per query and leaves rank * s keys
+    // (a tenth more for minima that share a slot) to insert.  Measured: c_pair 0.1 ps per
+    // pair of 64 packed BF16 elements (FP8 half, FP32 0.75 ps per 56); a key costs 37 ps
+    // where a tile of 32 references x 64 queries meets three of them and 80 ps where it
+    // meets one in two tiles (the tile leaves the short path for it alone), twice that for
+    // FP8.  The million-cell self search takes 174 / 152 / 146 / 146 ms with s = 2 / 4 / 8 /
+    // 16, the 100,000-cell one 2.91 / 2.68 / 2.67 / 2.87.
+    const double c_pair = dtype == SH_F32    ? 0.75e-12 * K / 56
+                          : dtype == SH_BF16 ? 0.1e-12 * K / 64
+                                             : 0.055e-12 * K / 64;
+    double best = 0.0;
+    for (int sh = 0; sh <= 4; ++sh) {
+      if (sh > 0 && (nr >> sh) < 8 * (int64_t)pool) break;
+      const int rank = p.collect ? tau_rank(pool, sh) : pool;
+      const double keys = 1.1 * rank * (1 << sh);
+      const double c_ins = (25e-12 + 75e-12 / (1.0 + keys * 2048.0 / (double)nr)) *
+                           (dtype == SH_FP8 ? 2.0 : 1.0);
+      const double cost = (double)nr * c_pair / (1 << sh) + keys * c_ins;
+      if (sh == 0 || cost < best) {
+        best = cost;
+        p.shift = sh;
+        p.rank = rank;
+      }
+    }
+    p.m = nr >> p.shift;
+    const int64_t res1 = (int64_t)std::max(1, ops.bound_resident ? ops.bound_resident(K) : 1) *
+                         kCUs;
+    const int max1 = (int)std::min<int64_t>(1024, cdiv(p.m, kSliceAlign));
+    // slots enough that the rank-th smallest minimum is close to the rank-th smallest key
+    const int min1 = (int)std::min<int64_t>(max1, cdiv(4 * (int64_t)p.rank, 16));
+    const int want1 = (int)std::min<int64_t>(max1, cdiv(res1, qb));
+    p.S1 = want1 > min1 ? want1 : pick_slices(qb, res1, min1, std::min(max1, min1 + 4));
+    p.len1 = align_up((size_t)cdiv(p.m, p.S1), kSliceAlign);
+    p.S1 = (int)cdiv(p.m, p.len1);
+    p.per = 16 * p.S1 <= 2048 ? 8 : 4 * p.S1 <= 2048 ? 2 : 1;
+    p.slots = p.S1 * 2 * p.per;
+    int64_t res3;
+    if (p.collect) {
+      res3 = (int64_t)std::max(1, ops.collect_resident ? ops.collect_resident(K) : 1) * kCUs;
+      // a query's keys vary with the sample by 1 / sqrt(rank); all may come from one slice
+      const double keys = 1.1 * p.rank * (1 << p.shift);
+      p.cap = (int)align_up((size_t)(keys * (1.0 + 5.5 / std::sqrt((double)p.rank))) + 64, 128);
+    } else {
+      res3 = (int64_t)std::max(1, ops.screen_resident ? ops.screen_resident(K, p.cap) : 1) *
+             kCUs;
+    }
+    // slices of at least 256 references, at most kBufBytes of candidate buffers
+    const int64_t room = std::max<int64_t>(
+        1, (int64_t)(kBufBytes / ((size_t)std::max<int64_t>(nq, 1) * p.cap * 8)));
+    const int max3 = (int)std::min<int64_t>(std::min<int64_t>(p.collect ? 256 : 1024, room),
+                                            std::max<int64_t>(1, nr / 256));
+    const int want3 = (int)cdiv(res3, qb);
+    p.S3 = want3 >= max3 ? max3
+                         : pick_slices(qb, res3, std::max(1, want3 - 1),
+                                       std::min(max3, want3 + 6));
+    p.len3 = align_up((size_t)cdiv(nr, p.S3), kSliceAlign);
+    p.S3 = (int)cdiv(nr, p.len3);
+  }
+  p.batch1 = std::min<int64_t>(
+      nq, std::max<int64_t>(256, (int64_t)(kSlotBytes / (std::max(p.slots, 1) * 4)) / 256 * 256));
+  p.batch3 = nq;
+  if (p.collect) {  // whole fills of the GPU a launch
+    const int64_t most = (int64_t)(kBufBytes / ((size_t)p.S3 * p.cap * 8));
+    const int64_t fill = (int64_t)ops.collect_resident(K) * kCUs * 256;
+    p.batch3 = std::min(nq, most >= fill ? most / fill * fill
+                                         : std::max<int64_t>(256, most / 256 * 256));
+  }
+  size_t o = align_up((size_t)nq * sizeof(float), 256);
+  p.off_slots = o;
+  if (p.bounded) o += align_up((size_t)p.batch1 * p.slots * sizeof(float), 256);
+  p.off_buf = o;
+  size_t keys = (size_t)p.batch3 * p.S3 * p.cap, segs = (size_t)p.batch3 * p.S3 * 2;
+  if (p.collect) {
+    const int cap2 = screen_cap(pool);
+    const int64_t n1 = std::min(nq, kAgain), n2 = std::min(std::max<int64_t>(nq - kAgain, 0),
+                                                           kAgainBatch);
+    keys = std::max(keys, (size_t)std::max(n1 * kAgainSlices, n2) * cap2);
+    segs = std::max(segs, (size_t)std::max(n1 * kAgainSlices, n2) * 2);
+  }
+  o += align_up(keys * sizeof(uint64_t), 256);
+  p.off_cnt = o;
+  if (p.collect || p.S3 > 1) o += align_up(segs * sizeof(int32_t), 256);
+  p.off_fail = o;
+  if (p.collect) o += 256 + align_up((size_t)nq * sizeof(int32_t), 256);
+  p.bytes = o;
+  return p;
+}
+
+struct MergeArgs {
+  const uint64_t *buf;
+  const int32_t *seg_cnt;
+  int64_t n;
+  int S, cap, pool, need;
+  const int32_t *list, *list_n;
+  int32_t list_base;
+  int32_t *fail, *fail_n;
+  int32_t fail_base;
+  uint64_t *out;
+  int32_t *out_cnt;
+};
+template <bool BITS>
+static void launch_merge(const MergeArgs &a, hipStream_t st) {
+  const dim3 grid((uint32_t)cdiv(a.n, 4));
+  const size_t lds = 4 * ((size_t)a.pool * sizeof(uint64_t) + 2 * (size_t)a.S * sizeof(int));
+#define SH_MERGE(PE, E)                                                                        \
+  hipLaunchKernelGGL((k_pool_merge<PE, E, BITS>), grid, dim3(256), lds, st, a.buf, a.seg_cnt, a.n,   \
+                     a.S, a.cap, a.pool, a.need, a.list, a.list_n, a.list_base, a.fail,        \
+                     a.fail_n, a.fail_base, a.out, a.out_cnt)
+  if (a.pool <= 64)
+    SH_MERGE(1, 8);
+  else if (a.pool <= 128)
+    SH_MERGE(2, 8);
+  else
+    SH_MERGE(4, 16);
+#undef SH_MERGE
+}
+}  // namespace sh
+
+extern "C" size_t sh_knn_pool_workspace(int64_t nq, int64_t nr, int32_t D, int dtype,
+                                        int32_t pool) {
+  if (nq <= 0 || nr <= 0 || D <= 0 || pool < 1 || pool > 256) return 0;
+  const int32_t K = pack_k(dtype, D);
+  return K > 0 ? pool_plan(nq, nr, K, dtype, pool).bytes : 0;
+}
+
+extern "C" int sh_knn_pool(const void *qpack, int64_t nq, const void *rpack, int64_t nr,
+                           int32_t D, int dtype, int32_t pool, uint64_t *cand_keys,
+                           int32_t *cand_cnt, void *workspace, size_t workspace_bytes,
+                           sh_stream_t stream) {
+  SH_ARG(nq >= 0 && nr > 0 && D > 0, "sh_knn_pool: bad sizes nq=%lld nr=%lld D=%d",
+         (long long)nq, (long long)nr, D);
+  SH_ARG(nr < 0xffffffffll, "sh_knn_pool: more than 2^32-1 references");
+  SH_ARG(nq <= 0x7fffffffll, "sh_knn_pool: too many queries");
+  SH_ARG(pool >= 1 && pool <= 256, "sh_knn_pool: pool=%d outside [1, 256]", pool);
+  SH_ARG(pool <= 128 || dtype == SH_FP8, "sh_knn_pool: pools above 128 are built for the FP8 "
+         "screen only (pool=%d)", pool);
+  SH_ARG(qpack && rpack && cand_keys && cand_cnt, "sh_knn_pool: NULL pointer");
+  const int32_t K = pack_k(dtype, D);
+  const KnnOps ops = knn_ops(dtype);
+  if (!ops.bound || K <= 0 || !ops.bound_resident(K)) {
+    set_error("sh_knn_pool: dtype %d with packed K=%d not supported", dtype, K);
+    return SH_EUNSUPPORTED;
+  }
+  if (nq == 0) return SH_OK;
+  const PoolPlan p = pool_plan(nq, nr, K, dtype, pool);
+  if (!workspace || workspace_bytes < p.bytes) {
+    set_error("sh_knn_pool: workspace %zu < %zu bytes", workspace_bytes, p.bytes);
+    return SH_EWORKSPACE;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  char *ws = (char *)workspace;
+  float *tau0 = (float *)ws;
+  float *slots = (float *)(ws + p.off_slots);
+  uint64_t *buf = (uint64_t *)(ws + p.off_buf);
+  int32_t *seg = (int32_t *)(ws + p.off_cnt);
+  int32_t *fail_n = (int32_t *)(ws + p.off_fail), *fail = fail_n + 64;
+  const int64_t qrow = pack_row_bytes(dtype, D);
+  if (p.bounded) {
+    for (int64_t q0 = 0; q0 < nq; q0 += p.batch1) {
+      const int64_t nb = std::min(p.batch1, nq - q0);
+      const BoundArgs b = {(const char *)qpack + q0 * qrow, nb,   rpack, p.m, p.shift, p.len1,
+                           p.S1,                            p.per, slots};
+      ops.bound(K, b, st);
+      SH_LAUNCH_CHECK("k_bound");
+      const dim3 grid((uint32_t)cdiv(nb, 4));
+#define SH_TAU(EL)                                                                           \
+  hipLaunchKernelGGL(k_tau<EL>, grid, dim3(256), 0, st, slots, nb, p.slots, p.rank, tau0 + q0, \
+                     p.collect && q0 == 0 ? fail_n : nullptr)
+      if (p.slots <= 64 * 2)
+        SH_TAU(2);
+      else if (p.slots <= 64 * 4)
+        SH_TAU(4);
+      else if (p.slots <= 64 * 8)
+        SH_TAU(8);
+      else
+        SH_TAU(32);
+#undef SH_TAU
+      SH_LAUNCH_CHECK("k_tau");
+    }
+  }
+  MergeArgs mg = {};
+  mg.buf = buf, mg.seg_cnt = seg, mg.pool = pool;
+  mg.need = (int)std::min<int64_t>(pool, nr);
+  mg.out = cand_keys, mg.out_cnt = cand_cnt;
+  ScreenArgs a = {};
+  a.q = qpack, a.r = rpack, a.nr = nr, a.pool = pool, a.buf = buf;
+  if (!p.collect) {
+    a.nq = nq, a.slice_len = p.len3, a.S = p.S3;
+    a.tau0 = p.bounded ? tau0 : nullptr;
+    a.seg_cnt = p.S3 > 1 ? seg : nullptr;
+    a.out = cand_keys, a.out_cnt = cand_cnt;
+    if (!ops.screen(K, p.cap, a, st)) {
+      set_error("sh_knn_pool: dtype %d with packed K=%d not supported", dtype, K);
+      return SH_EUNSUPPORTED;
+    }
+    SH_LAUNCH_CHECK("k_screen");
+    if (p.S3 > 1) {
+      mg.n = nq, mg.S = p.S3, mg.cap = p.cap;
+      launch_merge<false>(mg, st);
+      SH_LAUNCH_CHECK("k_pool_merge");
+    }
+    return SH_OK;
+  }
+  for (int64_t q0 = 0; q0 < nq; q0 += p.batch3) {
+    const int64_t nb = std::min(p.batch3, nq - q0);
+    const CollectArgs c = {(const char *)qpack + q0 * qrow, nb,    rpack, nr, p.len3, p.S3,
+                           tau0 + q0,                       p.cap, (uint2 *)buf, seg};
+    ops.collect(K, c, st);
+    SH_LAUNCH_CHECK("k_collect");
+    MergeArgs m = mg;
+    m.n = nb, m.S = p.S3, m.cap = p.cap;
+    m.fail = fail, m.fail_n = fail_n, m.fail_base = (int32_t)q0;
+    m.out = cand_keys + q0 * pool, m.out_cnt = cand_cnt + q0;
+    launch_merge<true>(m, st);
+    SH_LAUNCH_CHECK("k_pool_merge");
+  }
+  // the listed queries again, from an open threshold (their number stays on the device;
+  // workgroups past it leave at once)
+  for (int64_t base = 0; base < nq;) {
+    const bool first = base == 0;
+    const int64_t nb = std::min(nq - base, first ? kAgain : kAgainBatch);
+    const int S = first ? (int)std::max<int64_t>(1, std::min<int64_t>(kAgainSlices, nr / 256)) : 1;
+    a.nq = nb, a.slice_len = (int64_t)align_up((size_t)cdiv(nr, S), kSliceAlign);
+    a.S = (int)cdiv(nr, a.slice_len);
+    a.list = fail, a.list_n = fail_n, a.list_base = (int32_t)base;
+    a.seg_cnt = seg;
+    ops.screen(K, screen_cap(pool), a, st);
+    SH_LAUNCH_CHECK("k_screen");
+    MergeArgs m = mg;
+    m.n = nb, m.S = a.S, m.cap = screen_cap(pool);
+    m.list = fail, m.list_n = fail_n, m.list_base = (int32_t)base;
+    launch_merge<false>(m, st);
+    SH_LAUNCH_CHECK("k_pool_merge");
+    base += nb;
+  }
+  return SH_OK;
 }
 
 extern "C" int sh_knn_rerank(const float *Q, int64_t nq, int64_t ldq, const float *R, int64_t nr,

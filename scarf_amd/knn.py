@@ -169,10 +169,13 @@ def search(Q: "torch.Tensor", R: "torch.Tensor", refs: PackedRefs, k: int, pool:
     """Top-k of each query row of ``Q`` against ``R`` (both FP32 [*, D] on device).
 
     Returns (idx int64 [nq, k], dist f32 [nq, k], flags int32 [nq]).  ``order`` (default:
-    batches of at least ORDER_MIN_QUERIES rows) screens the queries in locality order;
-    with ``self_offset`` and ``seed``, each block of locality-ordered queries also seeds
-    the screen threshold with its own reference rows.  The results are the same either
-    way.
+    batches of at least ORDER_MIN_QUERIES rows) screens the queries in locality order.
+    Every query's pool comes from ``sh_knn_pool``: a pass over a sample of the references
+    bounds its threshold, then one scan collects what lies below.  ``n_slices`` asks for
+    the screen of ``sh_knn_screen`` instead, with an open threshold in each of so many
+    reference slices; there, with ``self_offset`` and ``seed``, each block of
+    locality-ordered queries seeds its threshold with its own reference rows.  The results
+    are the same either way.
 
     ``refine`` (default: on for the FP8 screen below a pool of REFINE_POOL): the re-rank
     flags queries whose k-th exact distance is not clear of the pool's cut-off by
@@ -258,15 +261,25 @@ def _search(Q, R, refs, k, pool, self_offset, n_slices, certify, self_idx, strea
     code = _lib.DTYPES[refs.dtype]
     st = stream_handle(stream)
     qp, _, _ = pack(Q, refs.dtype, 1, stream)
-    S = _fix_slices(nr, n_slices if n_slices else default_slices(nq, nr))
-    if S > 1:  # seeds pay off when every block sees all of its seed rows
-        seeds = None
-    cand = torch.empty((nq, S, pool), dtype=torch.int64, device=dev)
-    cnt = torch.empty((nq, S), dtype=torch.int32, device=dev)
-    ws, nbytes = workspace("screen").get(_lib.lib().sh_knn_screen_workspace(nq, pool, S))
-    with kernel_timer("screen", stream, flops=2.0 * nq * nr * D):
-        _lib.call("sh_knn_screen", ptr(qp), nq, ptr(refs.data), nr, D, code, None, None, pool,
-                  S, ptr(seeds), ptr(cand), ptr(cnt), ptr(ws), nbytes, st)
+    if n_slices:  # the caller's slice count: one pool per slice, merged in the re-rank
+        S = _fix_slices(nr, n_slices)
+        if S > 1:  # seeds pay off when every block sees all of its seed rows
+            seeds = None
+        cand = torch.empty((nq, S, pool), dtype=torch.int64, device=dev)
+        cnt = torch.empty((nq, S), dtype=torch.int32, device=dev)
+        ws, nbytes = workspace("screen").get(_lib.lib().sh_knn_screen_workspace(nq, pool, S))
+        with kernel_timer("screen", stream, flops=2.0 * nq * nr * D):
+            _lib.call("sh_knn_screen", ptr(qp), nq, ptr(refs.data), nr, D, code, None, None,
+                      pool, S, ptr(seeds), ptr(cand), ptr(cnt), ptr(ws), nbytes, st)
+    else:
+        S = 1
+        cand = torch.empty((nq, pool), dtype=torch.int64, device=dev)
+        cnt = torch.empty(nq, dtype=torch.int32, device=dev)
+        ws, nbytes = workspace("screen").get(
+            _lib.lib().sh_knn_pool_workspace(nq, nr, D, code, pool))
+        with kernel_timer("screen", stream, flops=2.0 * nq * nr * D):
+            _lib.call("sh_knn_pool", ptr(qp), nq, ptr(refs.data), nr, D, code, pool, ptr(cand),
+                      ptr(cnt), ptr(ws), nbytes, st)
     if certify is None:
         certify = refs.dtype in ("fp32", "f32")
     err_coef = -1.0

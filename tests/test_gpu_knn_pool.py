@@ -1,0 +1,105 @@
+"""sh_knn_pool (threshold pass, sliced scan, merge) keeps the pool that the one-slice screen
+with an open threshold keeps, bit for bit: it is the same set of MFMA keys, selected another
+way."""
+import sys
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def _rows(n, D, seed, dup=0):
+    rng = np.random.default_rng(seed)
+    c = rng.standard_normal((9, D)) * 2
+    E = (c[rng.integers(0, 9, n)] + rng.standard_normal((n, D))).astype(np.float32)
+    if dup:
+        E[rng.choice(n, min(dup, n), replace=False)] = E[0]
+    return E
+
+
+# query counts around a 256-query block, reference counts around the 128-row stage, the
+# smallest set that takes a threshold pass (8 pools) and one below it, several slices
+CASES = [("bf16", 64, 50, 1, 511), ("bf16", 64, 50, 1, 512), ("bf16", 64, 50, 33, 20001),
+         ("bf16", 64, 13, 257, 4097), ("bf16", 128, 70, 255, 9000), ("bf16", 64, 125, 40, 30000),
+         ("bf16", 64, 50, 3000, 60013), ("bf16", 32, 50, 9000, 9000),
+         ("fp32", 64, 50, 1, 40), ("fp32", 64, 50, 300, 19001), ("fp32", 128, 7, 65, 2049),
+         ("fp32", 16, 128, 31, 5000), ("fp8", 128, 100, 700, 30011), ("fp8", 64, 64, 1, 8192),
+         ("fp8", 256, 100, 130, 12000)]
+
+
+def _compare(Q, R, screen, pool):
+    """Pools of sh_knn_pool and of the one-slice open screen, as (keys, counts) pairs."""
+    import torch
+    from scarf_amd import _lib
+    from scarf_amd.device import ptr, stream_handle
+    from scarf_amd.knn import pack, pack_refs
+    L, code = _lib.lib(), _lib.DTYPES[screen]
+    (nq, D), nr = Q.shape, R.shape[0]
+    refs = pack_refs(R, screen)
+    qp, _, _ = pack(Q, screen, 1)
+    want = torch.full((nq, pool), -1, dtype=torch.int64, device="cuda")
+    want_n = torch.empty(nq, dtype=torch.int32, device="cuda")
+    ws = torch.empty(L.sh_knn_screen_workspace(nq, pool, 1), dtype=torch.uint8, device="cuda")
+    _lib.call("sh_knn_screen", ptr(qp), nq, ptr(refs.data), nr, D, code, None, None, pool, 1,
+              None, ptr(want), ptr(want_n), ptr(ws), ws.numel(), stream_handle())
+    got = torch.full_like(want, -1)
+    got_n = torch.empty_like(want_n)
+    ws = torch.empty(L.sh_knn_pool_workspace(nq, nr, D, code, pool), dtype=torch.uint8,
+                     device="cuda")
+    _lib.call("sh_knn_pool", ptr(qp), nq, ptr(refs.data), nr, D, code, pool, ptr(got),
+              ptr(got_n), ptr(ws), ws.numel(), stream_handle())
+    torch.cuda.synchronize()
+    assert torch.equal(got_n, want_n)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("screen,pool,D,nq,nr", CASES)
+@pytest.mark.parametrize("dup", [0, 400])
+def test_pool_equals_open_screen(cuda, screen, pool, D, nq, nr, dup):
+    import torch
+    say("knn pool", screen, "pool", pool, "D", D, nq, "x", nr, "dup", dup)
+    R = torch.from_numpy(_rows(nr, D, 5, dup)).cuda()
+    Q = torch.from_numpy(_rows(nq, D, 6)).cuda()
+    if dup:
+        Q[0] = R[0]  # a query whose nearest keys are all equal
+    _compare(Q, R, screen, pool)
+
+
+# over a billion pairs: the collecting scan, whose overflowing queries (a thousand equal
+# references each, more of them than the first list of the second screen takes) are
+# screened again
+@pytest.mark.parametrize("screen,pool,D,nq,nr,equal", [
+    ("bf16", 64, 50, 9001, 120_013, 0), ("bf16", 64, 50, 13_000, 100_000, 6_000),
+    ("bf16", 128, 20, 20_000, 60_001, 3), ("fp32", 64, 50, 20_011, 55_000, 700),
+    ("fp8", 128, 100, 9_000, 131_072, 40), ("fp8", 256, 100, 3_001, 400_000, 1)])
+def test_collected_pool_equals_open_screen(cuda, screen, pool, D, nq, nr, equal):
+    import torch
+    say("knn collect", screen, "pool", pool, "D", D, nq, "x", nr, "equal", equal)
+    R = torch.from_numpy(_rows(nr, D, 7, 3000 if equal else 0)).cuda()
+    Q = torch.from_numpy(_rows(nq, D, 8)).cuda()
+    Q[:equal] = R[0]
+    _compare(Q, R, screen, pool)
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3, 4])
+def test_misleading_sample(cuda, shift):
+    """Near references only where the threshold pass looks: its guess is too low, the scan
+    meets fewer keys than the pool, and the query is screened again."""
+    import torch
+    say("knn misleading sample", shift)
+    nr, nq, D, near = 120_000, 9_000, 50, 60
+    i = np.arange(near, dtype=np.uint64) * 31
+    rows = (i << np.uint64(shift)) + ((((i * np.uint64(2654435761)) & np.uint64(0xffffffff))
+                                       >> np.uint64(16)) & np.uint64((1 << shift) - 1))
+    E = _rows(nr, D, 9)
+    rng = np.random.default_rng(10)
+    E[rows.astype(np.int64)] = 40.0 + 0.01 * rng.standard_normal((near, D))
+    Q = _rows(nq, D, 11)
+    Q[100:5000] = 40.0 + 0.01 * rng.standard_normal((4900, D))
+    _compare(torch.from_numpy(Q.astype(np.float32)).cuda(), torch.from_numpy(E).cuda(), "bf16", 64)
