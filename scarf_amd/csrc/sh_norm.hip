@@ -8,6 +8,7 @@
 #include <float.h>
 
 #include <algorithm>
+#include <utility>
 
 #include "sh_common.h"
 
@@ -258,7 +259,45 @@ __global__ void __launch_bounds__(256) k_densify(
 // FP32 accumulators.  Each group thus gathers a whole W row per load instruction; the
 // groups' sums are added in a fixed order at the end of the row.  DPL = 64-column
 // passes (D <= 64 * DPL).
+//
+// The gathers are the traffic (a W row per non-zero, from L2), and what bounds it is the
+// L1's share of them: eight gathers in flight a wave instead of one, rows padded to whole
+// cache lines, and 32-bit row offsets each changed nothing.  A group's own lanes hold its
+// entries (lane i of group g: entry 4 i + g of the batch), so an entry reaches its group by
+// a DPP row broadcast instead of ds_bpermute; the next batch's counts are in flight during
+// this one's gathers.  500,000 x 2000 at 8% non-zeros, D = 50: 1622 -> 1327 us.
 constexpr int kProjGroup = 16;
+template <int I>
+__device__ __forceinline__ int row_bcast(int v) {  // lane I of each 16-lane row
+  return __builtin_amdgcn_update_dpp(0, v, 0x150 + I, 0xF, 0xF, true);
+}
+template <int DPL, int I>
+__device__ __forceinline__ void project_step(int f, float delta, int cnt, int c4,
+                                             const bool (&col_ok)[DPL], const float4 *W4,
+                                             uint32_t ld4, float4 (&acc)[DPL]) {
+  if (4 * I >= cnt) return;  // the same for the whole wave
+  const int fj = row_bcast<I>(f);
+  const float dj = __int_as_float(row_bcast<I>(__float_as_int(delta)));
+  if (fj >= 0) {
+#pragma unroll
+    for (int p = 0; p < DPL; ++p) {
+      if (col_ok[p]) {
+        const float4 w = W4[(uint64_t)(uint32_t)fj * ld4 + c4 + kProjGroup * p];
+        acc[p].x = fmaf(dj, w.x, acc[p].x);
+        acc[p].y = fmaf(dj, w.y, acc[p].y);
+        acc[p].z = fmaf(dj, w.z, acc[p].z);
+        acc[p].w = fmaf(dj, w.w, acc[p].w);
+      }
+    }
+  }
+}
+template <int DPL, int... I>
+__device__ __forceinline__ void project_batch(std::integer_sequence<int, I...>, int f,
+                                              float delta, int cnt, int c4,
+                                              const bool (&col_ok)[DPL], const float4 *W4,
+                                              uint32_t ld4, float4 (&acc)[DPL]) {
+  (project_step<DPL, I>(f, delta, cnt, c4, col_ok, W4, ld4, acc), ...);
+}
 template <int DPL>
 __global__ void __launch_bounds__(256) k_project(
     const uint32_t *__restrict__ vals, const int32_t *__restrict__ cols,
@@ -283,7 +322,7 @@ __global__ void __launch_bounds__(256) k_project(
     l = s == 0 ? 1.0 : (double)s;
   }
   const float scale = sf / (float)l;
-  const int64_t ld4 = ldw / 4;
+  const uint32_t ld4 = (uint32_t)(ldw / 4);
   const float4 *W4 = reinterpret_cast<const float4 *>(W);
   bool col_ok[DPL];
 #pragma unroll
@@ -291,15 +330,28 @@ __global__ void __launch_bounds__(256) k_project(
   float4 acc[DPL];
 #pragma unroll
   for (int p = 0; p < DPL; ++p) acc[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int mine = 4 * c4 + grp;  // this lane's entry of a batch
+  int32_t c = -1;
+  uint32_t v = 0;
+  if (a + mine < b) {
+    c = cols[a + mine];
+    v = vals[a + mine];
+  }
   for (int64_t t0 = a; t0 < b; t0 += 64) {
-    const int64_t t = t0 + lane;
+    const int64_t tn = t0 + 64 + mine;
+    int32_t cn = -1;
+    uint32_t vn = 0;
+    if (tn < b) {
+      cn = cols[tn];
+      vn = vals[tn];
+    }
     int f = -1;
     float delta = 0.f;
-    if (t < b) {
-      f = map_col(col_map, cols[t], n_in);
+    if (t0 + mine < b) {
+      f = map_col(col_map, c, n_in);
       if (f >= 0) {
-        const float v = (float)vals[t] * scale;
-        const float xv = log_t ? log1pf(v) : v;
+        const float x = (float)v * scale;
+        const float xv = log_t ? log1pf(x) : x;
         if (clip > 0.f) {
           const float zs = (xv - mu[f]) * inv_sigma[f];
           const float z0 = (0.f - mu[f]) * inv_sigma[f];
@@ -309,28 +361,10 @@ __global__ void __launch_bounds__(256) k_project(
         }
       }
     }
-    // The trip count is the same for the whole wave, so every lane takes part in every
-    // shuffle (a shuffle from a lane that has left the loop reads 0); lanes past the row's
-    // end hold f = -1 and add nothing.
-    const int cnt = (int)min<int64_t>(64, b - t0);
-#pragma unroll 4
-    for (int j0 = 0; j0 < cnt; j0 += 64 / kProjGroup) {
-      const int j = j0 + grp;
-      const int fj = __shfl(f, j, 64);
-      const float dj = __shfl(delta, j, 64);
-      if (fj >= 0) {
-#pragma unroll
-        for (int p = 0; p < DPL; ++p) {
-          if (col_ok[p]) {
-            const float4 w = W4[(int64_t)fj * ld4 + c4 + kProjGroup * p];
-            acc[p].x = fmaf(dj, w.x, acc[p].x);
-            acc[p].y = fmaf(dj, w.y, acc[p].y);
-            acc[p].z = fmaf(dj, w.z, acc[p].z);
-            acc[p].w = fmaf(dj, w.w, acc[p].w);
-          }
-        }
-      }
-    }
+    project_batch<DPL>(std::make_integer_sequence<int, kProjGroup>{}, f, delta,
+                       (int)min<int64_t>(64, b - t0), c4, col_ok, W4, ld4, acc);
+    c = cn;
+    v = vn;
   }
   // groups 0 + 1 and 2 + 3, then the two pairs
 #pragma unroll
