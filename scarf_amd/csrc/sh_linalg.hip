@@ -99,24 +99,109 @@ __global__ void __launch_bounds__(256) k_dgemm(int transA, int64_t m, int64_t n,
       }
 }
 
+// C[m x n] = alpha A B + beta C for a tall A (m x k) and a small B, k and n at most
+// kTallMax: the block times the b x b matrices of the subspace iteration.  Wave (x, y) of the
+// grid computes 16 rows x 16 columns; both operands come straight from memory (B from L2),
+// eight k-steps of loads in flight before their MFMAs, no LDS and no barriers.  The 64 x 64
+// tiles of k_dgemm give such a product 64 workgroups that wait for each 16-step stage:
+// 2000 x 94 x 94 took 32 us, here 10.5.  The products are added in the same order.
+constexpr int kTallMax = 256;
+constexpr int kTallU = 8;
+__global__ void __launch_bounds__(256) k_dgemm_tall(int64_t m, int32_t n, int32_t k,
+                                                    const double *__restrict__ A, int64_t lda,
+                                                    const double *__restrict__ B, int64_t ldb,
+                                                    double alpha, double beta,
+                                                    double *__restrict__ C, int64_t ldc) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int kr = lane >> 4, cl = lane & 15;
+  const int64_t m0 = (int64_t)blockIdx.x * 16;
+  const int n0 = (int)(blockIdx.y * 4 + w) * 16;
+  if (n0 >= n) return;
+  const bool row_ok = m0 + cl < m, col_ok = n0 + cl < n;
+  const double *Ar = A + (m0 + cl) * lda;
+  const double *Bc = B + n0 + cl;
+  doublex4 acc = {0.0, 0.0, 0.0, 0.0};
+  for (int k0 = 0; k0 < k; k0 += 4 * kTallU) {
+    double a[kTallU], b[kTallU];
+#pragma unroll
+    for (int u = 0; u < kTallU; ++u) {
+      const int kk = k0 + 4 * u + kr;
+      a[u] = (row_ok && kk < k) ? Ar[kk] : 0.0;
+      b[u] = (col_ok && kk < k) ? Bc[(int64_t)kk * ldb] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < kTallU; ++u)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[u], acc, 0, 0, 0);
+  }
+  if (!col_ok) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int64_t row = m0 + 4 * i + kr;
+    if (row < m) {
+      double v = alpha * acc[i];
+      if (beta != 0.0) v += beta * C[row * ldc + n0 + cl];
+      C[row * ldc + n0 + cl] = v;
+    }
+  }
+}
+
 // ---- merge matrix of one partial fit ------------------------------------------------
 // M = (G - n bm bm^T) + Vt^T diag(s2) Vt + mc mc^T, every term formed so that M[i][j] and
 // M[j][i] round identically (G is stored symmetric).
-__global__ void k_merge_matrix(const double *__restrict__ G, int32_t d, double n,
-                               const double *__restrict__ bm, const double *__restrict__ Vt,
-                               const double *__restrict__ s2, int32_t nc,
-                               const double *__restrict__ mc, double *__restrict__ M) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)d * d) return;
-  const int i = (int)(e / d), j = (int)(e % d);
-  double v = G[e] - n * (bm[i] * bm[j]);
+//
+// 64 x 64 entries per workgroup, 4 x 4 per thread, the two 64-column strips of Vt in LDS
+// kMmC rows at a time: one thread per entry re-read both strips for every entry (166 us at
+// d = 2000, 51 components; now about 30).
+constexpr int kMmT = 64, kMmC = 32;
+__global__ void __launch_bounds__(256) k_merge_matrix(
+    const double *__restrict__ G, int32_t d, double n, const double *__restrict__ bm,
+    const double *__restrict__ Vt, const double *__restrict__ s2, int32_t nc,
+    const double *__restrict__ mc, double *__restrict__ M) {
+  __shared__ double vi[kMmC][kMmT], vj[kMmC][kMmT];
+  const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
+  const int i0 = blockIdx.y * kMmT, j0 = blockIdx.x * kMmT;
+  double r[4][4] = {};
   if (Vt) {
-    double r = 0.0;
-    for (int c = 0; c < nc; ++c) r += s2[c] * (Vt[(int64_t)c * d + i] * Vt[(int64_t)c * d + j]);
-    v += r;
+    for (int c0 = 0; c0 < nc; c0 += kMmC) {
+      const int cn = min(kMmC, nc - c0);
+      for (int e = tid; e < cn * kMmT; e += 256) {
+        const int c = e / kMmT, t = e % kMmT;
+        const double *row = Vt + (int64_t)(c0 + c) * d;
+        vi[c][t] = i0 + t < d ? row[i0 + t] : 0.0;
+        vj[c][t] = j0 + t < d ? row[j0 + t] : 0.0;
+      }
+      __syncthreads();
+      for (int c = 0; c < cn; ++c) {
+        const double sc = s2[c0 + c];
+        double a[4], b[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          a[u] = vi[c][ty + 16 * u];
+          b[u] = vj[c][tx + 16 * u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) r[u][v] += sc * (a[u] * b[v]);
+      }
+      __syncthreads();
+    }
   }
-  if (mc) v += mc[i] * mc[j];
-  M[e] = v;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int i = i0 + ty + 16 * u;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int j = j0 + tx + 16 * v;
+      if (i < d && j < d) {
+        const int64_t e = (int64_t)i * d + j;
+        double x = G[e] - n * (bm[i] * bm[j]);
+        if (Vt) x += r[u][v];
+        if (mc) x += mc[i] * mc[j];
+        M[e] = x;
+      }
+    }
+  }
 }
 
 // ---- block Lanczos pieces -------------------------------------------------------------
@@ -480,7 +565,9 @@ template <int NT>
 __global__ void __launch_bounds__(256) k_symm_block_part(
     const double *__restrict__ M, int32_t d, const double *__restrict__ Y, int64_t ldy,
     int32_t kslice, double *__restrict__ part /* [slices][d][ldy] */) {
-  __shared__ double ys[2][kSbK][16 * NT];
+  // an even NT's rows are a multiple of 64 banks long: 16 doubles more put the two rows that a
+  // half wave reads on different banks
+  __shared__ double ys[2][kSbK][16 * NT + (NT % 2 ? 0 : 16)];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int kr = lane >> 4, cl = lane & 15;
   const int64_t row = (int64_t)blockIdx.x * kSbRows + 16 * w + cl;  // this lane's A row
@@ -568,7 +655,8 @@ __global__ void __launch_bounds__(256) k_symm_block_sum(
 // row-major): the rows are split into slices, each workgroup computes one 64 x 64 output
 // block of one slice (four waves of 32 x 32, v_mfma_f64_16x16x4f64, operands read
 // straight from memory: each lane quarter reads 16 consecutive doubles of one row), and
-// k_block_gram_sum adds the slices in slice order.
+// k_block_gram_sum adds the slices in a fixed order: eight interleaved sums per entry, a
+// thread each (one thread walking all 125 slices took 32 us at 94 x 94; now 4.3).
 constexpr int kBgSlices = 128;
 __global__ void __launch_bounds__(256) k_block_gram_part(
     const double *__restrict__ A, int64_t lda, int32_t na, const double *__restrict__ B,
@@ -617,13 +705,22 @@ __global__ void __launch_bounds__(256) k_block_gram_part(
       }
 }
 
-__global__ void k_block_gram_sum(const double *__restrict__ part, int32_t slices, int32_t n,
-                                 double *__restrict__ C) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
+constexpr int kBgElems = 32, kBgParts = 8;
+__global__ void __launch_bounds__(kBgElems *kBgParts) k_block_gram_sum(
+    const double *__restrict__ part, int32_t slices, int32_t n, double *__restrict__ C) {
+  __shared__ double sums[kBgParts][kBgElems];
+  const int te = threadIdx.x % kBgElems, u = threadIdx.x / kBgElems;
+  const int64_t e = (int64_t)blockIdx.x * kBgElems + te;
   double s = 0.0;
-  for (int t = 0; t < slices; ++t) s += part[(int64_t)t * n + e];
-  C[e] = s;
+  if (e < n) {
+#pragma unroll 4
+    for (int t = u; t < slices; t += kBgParts) s += part[(int64_t)t * n + e];
+  }
+  sums[u][te] = s;
+  __syncthreads();
+  if (u == 0 && e < n)
+    C[e] = ((sums[0][te] + sums[1][te]) + (sums[2][te] + sums[3][te])) +
+           ((sums[4][te] + sums[5][te]) + (sums[6][te] + sums[7][te]));
 }
 
 // res[c] = || XM[:, c] - theta[c] X[:, c] || for c < b: one workgroup per column, the
@@ -731,8 +828,8 @@ extern "C" int sh_block_gram(const double *A, int64_t lda, int32_t na, const dou
   hipLaunchKernelGGL(k_block_gram_part, dim3((uint32_t)slices, (uint32_t)blocks), dim3(256), 0,
                      st, A, lda, na, B, ldb, nb, d, rps, part);
   const int64_t n = (int64_t)na * nb;
-  hipLaunchKernelGGL(k_block_gram_sum, dim3((uint32_t)cdiv(n, 256)), dim3(256), 0, st, part,
-                     (int32_t)slices, (int32_t)n, C);
+  hipLaunchKernelGGL(k_block_gram_sum, dim3((uint32_t)cdiv(n, kBgElems)),
+                     dim3(kBgElems * kBgParts), 0, st, part, (int32_t)slices, (int32_t)n, C);
   SH_LAUNCH_CHECK("sh_block_gram");
   return SH_OK;
 }
@@ -757,6 +854,14 @@ extern "C" int sh_dgemm(int transA, int64_t m, int64_t n, int64_t k, double alph
          "sh_dgemm: leading dimension too small");
   SH_ARG(cdiv(n, kDT) <= 0x7fffffff && cdiv(m, kDT) <= 65535, "sh_dgemm: matrix too large");
   if (m == 0 || n == 0) return SH_OK;
+  // narrow products of many rows; below that (or wider) the 64 x 64 tiles fill the GPU
+  if (!transA && n <= kTallMax && k <= kTallMax && m >= 256 && cdiv(m, 16) <= 0x7fffffff) {
+    hipLaunchKernelGGL(k_dgemm_tall, dim3((uint32_t)cdiv(m, 16), (uint32_t)cdiv(n, 64)),
+                       dim3(256), 0, (hipStream_t)stream, m, (int32_t)n, (int32_t)k, A, lda, B,
+                       ldb, alpha, beta, C, ldc);
+    SH_LAUNCH_CHECK("k_dgemm_tall");
+    return SH_OK;
+  }
   dim3 grid((uint32_t)cdiv(n, kDT), (uint32_t)cdiv(m, kDT));
   hipLaunchKernelGGL(k_dgemm, grid, dim3(256), 0, (hipStream_t)stream, transA, m, n, k, A, lda,
                      B, ldb, alpha, beta, C, ldc);
@@ -769,9 +874,9 @@ extern "C" int sh_merge_matrix(const double *G, int32_t d, double n, const doubl
                                double *M, sh_stream_t stream) {
   SH_ARG(d > 0 && G && bm && M, "sh_merge_matrix: bad arguments");
   SH_ARG(!Vt || (s2 && nc > 0), "sh_merge_matrix: Vt needs s2 and nc > 0");
-  const int64_t n2 = (int64_t)d * d;
-  hipLaunchKernelGGL(k_merge_matrix, dim3((uint32_t)cdiv(n2, 256)), dim3(256), 0,
-                     (hipStream_t)stream, G, d, n, bm, Vt, s2, nc, mc, M);
+  const uint32_t t = (uint32_t)cdiv(d, kMmT);
+  hipLaunchKernelGGL(k_merge_matrix, dim3(t, t), dim3(256), 0, (hipStream_t)stream, G, d, n, bm,
+                     Vt, s2, nc, mc, M);
   SH_LAUNCH_CHECK("k_merge_matrix");
   return SH_OK;
 }
