@@ -274,8 +274,18 @@ def chebyshev_subspace(dev, n_top: int, tol: float, dyn: float = 16.0,
     [0, cut] (the merge matrix is positive semi-definite; cut is the block's smallest
     Ritz value) and is scaled to 1 at an upper bound of the active spectrum, then takes
     one CholeskyQR pass and the Ritz pairs of the generalized problem H q = theta G q (G the
-    block's Gram after that pass, so a second pass is not needed).  The degree is chosen so
-    that the filtered block's condition number stays below e^dyn.  Leading pairs whose
+    block's Gram after that pass, so a second pass is not needed).
+
+    The degree is as high as the Cholesky step can take, since an iteration's host round
+    trip costs some 25 filter steps.  Filtering grows column j by p(theta_j), which a
+    Cholesky factorisation does not mind (it is accurate to the condition number of the
+    column-scaled Gram); what matters is how much of the larger directions each column
+    holds.  A Ritz vector's share of direction i is below e_i = res_i / (theta_i - cut), so
+    the scaled block's condition number stays near e^dyn for
+    m <= (dyn + 0.8 ln(1 / e_i)) / acosh(x_i) (0.8: the residuals are estimates).  And it is
+    no higher than the wanted pairs need to reach a hundredth of the tolerance.  Against a
+    bound of dyn / acosh(x_1) this takes 5-6 iterations instead of 7-8 at the same number
+    of filter steps.  Leading pairs whose
     residual is far below the tolerance (so that removing them perturbs the rest by less
     than lock_factor * tol * theta_max) are locked and deflated out of the working
     matrix, which shrinks the dynamic range of the next filters: the well separated top
@@ -321,8 +331,13 @@ def chebyshev_subspace(dev, n_top: int, tol: float, dyn: float = 16.0,
         if not (cut > 0.0 and lam_up > cut):
             raise EigenNotConverged(f"degenerate filter interval (cut {cut:.3e}, top {lam_up:.3e})")
         half = 0.5 * cut
-        x_up = (lam_up - half) / half
-        m = int(dyn / math.acosh(max(x_up, 1.0 + 1e-12)))
+        x = np.maximum((th - half) / half, 1.0 + 1e-12)
+        x[0] = max(x[0], (lam_up - half) / half)
+        rate = np.arccosh(x)
+        share = np.clip(res / np.maximum(th - cut, 1e-16 * th[0]), 1e-14, 1.0)
+        m = int(np.min((dyn - 0.8 * np.log(share)) / rate))
+        left = np.log(np.maximum(res[:need] / (0.01 * thr), 1.0)) / rate[:need]
+        m = min(m, int(np.ceil(np.max(left))) + 1)
         m = max(2, min(max_degree if res[0] <= 1e-3 * th[0] else 4, m))
         dev.filter(m, half, half, lam_up)
         # one CholeskyQR pass, then the Rayleigh-Ritz step as H q = theta G q with the
@@ -388,9 +403,8 @@ class _DeviceBlock:
         self.L = torch.empty((n_top, self.d), dtype=torch.float64, device=dv)
         self.T = torch.empty((n_top, self.d), dtype=torch.float64, device=dv)
         self.theta_l = np.zeros(0)
-        self.th_dev = torch.zeros(self.ld, dtype=torch.float64, device=dv)
         self.res_dev = torch.zeros(self.ld, dtype=torch.float64, device=dv)
-        self.G = torch.empty((self.ld, self.ld), dtype=torch.float64, device=dv)
+        self.G = torch.empty(2 * self.ld * self.ld, dtype=torch.float64, device=dv)
         L = _lib.lib()
         # the k-slice count grows as the block shrinks: size for the narrowest block
         self.ws_sb, self.nb_sb = workspace("chfsi_sb").get(
@@ -408,17 +422,27 @@ class _DeviceBlock:
     def _cols(self) -> int:
         return _block_ld(self.nb)
 
-    def _gram(self, A, B, n):
-        _lib.call("sh_block_gram", ptr(A), self.ld, n, ptr(B), self.ld, n, self.d, ptr(self.G),
-                  ptr(self.ws_g), self.nb_g, self.st)
-        return self.G.view(-1)[:n * n].view(n, n)
+    def _gram(self, A, B, n, slot=0):
+        """A^T B of the first n columns, in the slot-th n x n part of self.G."""
+        _lib.call("sh_block_gram", ptr(A), self.ld, n, ptr(B), self.ld, n, self.d,
+                  ptr(self.G, slot * n * n), ptr(self.ws_g), self.nb_g, self.st)
 
-    def _times_small(self, A, S: np.ndarray, out):
-        """out[:, :n] = A[:, :k] S for a host matrix S (k x n)."""
-        k, n = S.shape
-        S_dev = torch.from_numpy(np.ascontiguousarray(S)).to(self.M.device)
-        _lib.call("sh_dgemm", 0, self.d, n, k, 1.0, ptr(A), self.ld, ptr(S_dev), n, 0.0,
+    def _grams(self, count, n) -> np.ndarray:
+        """The first ``count`` n x n Grams on the host, in one copy."""
+        return self.G[:count * n * n].cpu().numpy().reshape(count, n, n)
+
+    def _times_small(self, A, S_dev, n, out):
+        """out[:, :n] = A[:, :n] S for a device matrix S (n x n)."""
+        _lib.call("sh_dgemm", 0, self.d, n, n, 1.0, ptr(A), self.ld, ptr(S_dev), n, 0.0,
                   ptr(out), self.ld, self.st)
+
+    def _upload(self, a: np.ndarray):
+        return torch.from_numpy(np.ascontiguousarray(a)).to(self.M.device)
+
+    def _residuals(self, X, XM, w_dev, n) -> np.ndarray:
+        _lib.call("sh_block_residual", ptr(X), ptr(XM), self.d, n, self.ld, ptr(w_dev),
+                  ptr(self.res_dev), self.st)
+        return self.res_dev[:n].cpu().numpy()
 
     def _spare(self, *used):
         for i in range(len(self.buf)):
@@ -429,19 +453,17 @@ class _DeviceBlock:
     def _cholqr_pass(self):
         n = self.nb
         X = self.buf[self.X]
-        G = self._gram(X, X, n).cpu().numpy()
+        self._gram(X, X, n)
+        G = self._grams(1, n)[0]
         G = 0.5 * (G + G.T)
-        try:
-            with _one_thread():
-                R = _sla.cholesky(G, lower=False)  # G = R^T R (scipy: see rayleigh_ritz)
-        except np.linalg.LinAlgError as exc:
-            raise EigenNotConverged("filtered block lost rank (CholeskyQR)") from exc
-        with _one_thread():
-            Rinv, info = _sla.lapack.dtrtri(R, lower=0)
-        if info != 0:
+        with _one_thread():  # G = R^T R (scipy: see rayleigh_ritz)
+            R, info = _sla.lapack.dpotrf(G, lower=0)
+            if info == 0:
+                Rinv, info = _sla.lapack.dtrtri(R, lower=0)
+        if info != 0 or not np.all(np.isfinite(Rinv)):
             raise EigenNotConverged("filtered block lost rank (CholeskyQR)")
         o = self._spare(self.X)
-        self._times_small(X, Rinv, self.buf[o])
+        self._times_small(X, self._upload(Rinv), n, self.buf[o])
         self.X = o
 
     def orthonormalize(self):
@@ -459,31 +481,31 @@ class _DeviceBlock:
         XM = self.buf[xm]
         _lib.call("sh_symm_block", ptr(self.Mw), self.d, ptr(X), None, cols, self.ld, 1.0, 0.0,
                   0.0, ptr(XM), ptr(self.ws_sb), self.nb_sb, self.st)
-        Hd = self._gram(X, XM, n).clone()
-        if generalized:  # the block's own Gram, read back with H in one copy
-            Gd = self._gram(X, X, n)
-            HG = torch.cat([Hd, Gd]).cpu().numpy()
-            H, G = HG[:n], HG[n:]
-        else:
-            H, G = Hd.cpu().numpy(), None
+        self._gram(X, XM, n)
+        if generalized:  # the block's own Gram too, read back with H in one copy
+            self._gram(X, X, n, slot=1)
+        HG = self._grams(2 if generalized else 1, n)
+        HG = 0.5 * (HG + HG.transpose(0, 2, 1))
+        if not np.all(np.isfinite(HG)):
+            raise EigenNotConverged("filtered block lost rank (Rayleigh-Ritz)")
         # scipy's LAPACK binding: numpy's eigh and cholesky are an order of magnitude
         # slower at these sizes on a many-threaded host
         try:
             with _one_thread():
-                w, Q = _sla.eigh(0.5 * (H + H.T), None if G is None else 0.5 * (G + G.T),
-                                 driver="evd" if G is None else "gvd")
+                w, Q = _sla.eigh(HG[0], HG[1] if generalized else None,
+                                 driver="gvd" if generalized else "evd", check_finite=False,
+                                 overwrite_a=True, overwrite_b=True)
         except np.linalg.LinAlgError as exc:
             raise EigenNotConverged("filtered block lost rank (Rayleigh-Ritz)") from exc
-        w, Q = w[::-1].copy(), np.ascontiguousarray(Q[:, ::-1])
+        w = w[::-1].copy()
+        up = self._upload(np.concatenate([Q[:, ::-1].ravel(), w]))  # Q and theta, one copy
+        w_dev = up[n * n:]
         xo = self._spare(self.X, xm)
         mo = self._spare(self.X, xm, xo)
-        self._times_small(X, Q, self.buf[xo])
-        self._times_small(XM, Q, self.buf[mo])
-        self.th_dev[:n].copy_(torch.from_numpy(w))
-        _lib.call("sh_block_residual", ptr(self.buf[xo]), ptr(self.buf[mo]), self.d, n, self.ld,
-                  ptr(self.th_dev), ptr(self.res_dev), self.st)
+        self._times_small(X, up, n, self.buf[xo])
+        self._times_small(XM, up, n, self.buf[mo])
         self.X = xo
-        return w, self.res_dev[:n].cpu().numpy()
+        return w, self._residuals(self.buf[xo], self.buf[mo], w_dev, n)
 
     def lock(self, c: int, theta: np.ndarray):
         nl = self.theta_l.shape[0]
@@ -526,13 +548,31 @@ class _DeviceBlock:
         self.X = y1
 
     def result(self, n_active: int):
+        """The locked and leading active pairs against the original matrix: Rayleigh
+        quotients (descending), rows, the largest relative residual and the orthogonality
+        defect, all from the block kernels; only the rows themselves and n x n products
+        come to the host."""
         nl = self.theta_l.shape[0]
-        n_top = nl + n_active
-        Vt = torch.empty((n_top, self.d), dtype=torch.float64, device=self.M.device)
+        n = nl + n_active
+        vo = self._spare(self.X)
+        mo = self._spare(self.X, vo)
+        V, VM = self.buf[vo], self.buf[mo]
+        V.zero_()
         if nl:
-            Vt[:nl].copy_(self.L[:nl])
-        Vt[nl:].copy_(self.buf[self.X][:, :n_active].t())
-        return _verify_rows(self.M, Vt, self.d, self.st)
+            V[:, :nl].copy_(self.L[:nl].t())
+        V[:, nl:n].copy_(self.buf[self.X][:, :n_active])
+        _lib.call("sh_symm_block", ptr(self.M), self.d, ptr(V), None, _block_ld(n), self.ld, 1.0,
+                  0.0, 0.0, ptr(VM), ptr(self.ws_sb), self.nb_sb, self.st)
+        self._gram(V, VM, n)
+        self._gram(V, V, n, slot=1)
+        HG = self._grams(2, n)
+        theta = np.diagonal(HG[0]).copy()
+        res = self._residuals(V, VM, self._upload(theta), n)
+        Vh = V[:, :n].t().contiguous().cpu().numpy()
+        order = np.argsort(-theta, kind="stable")
+        scale = max(abs(theta[order[0]]), np.finfo(float).tiny)
+        orth = float(np.max(np.abs(HG[1] - np.eye(n))))
+        return theta[order], Vh[order], float(np.max(res)) / scale, orth
 
 
 def _verify_rows(M, Vt, d, st):
