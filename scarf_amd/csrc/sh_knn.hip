@@ -37,142 +37,145 @@ int64_t pack_row_bytes(int dtype, int32_t D) {
   return (int64_t)K + 16;
 }
 
-// float -> OCP FP8 E4M3 (bias 7, max 448, no infinities), round to nearest even,
-// saturating at +-448.
-__device__ __forceinline__ uint8_t f2e4m3(float x) {
-  const uint32_t sign = (__float_as_uint(x) >> 24) & 0x80u;
-  const float a = fabsf(x);
-  if (!(a == a)) return (uint8_t)(sign | 0x7Fu);
-  if (a >= 464.0f) return (uint8_t)(sign | 0x7Eu);
-  if (a < 0.015625f) {  // subnormal: multiples of 2^-9 (8 -> the smallest normal)
-    const int m = (int)rintf(a * 512.0f);
-    return (uint8_t)(sign | (uint32_t)m);
-  }
-  int e;
-  frexpf(a, &e);                              // a = f * 2^e, f in [0.5, 1)
-  int E = e - 1 + 7;                          // biased exponent of 1.m * 2^(e-1)
-  int m = (int)rintf((ldexpf(a, 1 - e) - 1.0f) * 8.0f);
-  if (m == 8) {
-    m = 0;
-    ++E;
-  }
-  if (E > 15 || (E == 15 && m == 7)) return (uint8_t)(sign | 0x7Eu);
-  return (uint8_t)(sign | ((uint32_t)E << 3) | (uint32_t)m);
-}
-
-// FP8 rows: x / 2^e in E4M3 with e the smallest power of two that brings max|x|
-// under 448; role 0 packs r and its ||r||^2, role 1 packs -2q.
-__global__ void k_pack_fp8(const float *__restrict__ E, int64_t n, int32_t D, int64_t lde,
-                           int role, int32_t K, uint8_t *__restrict__ out,
-                           float *__restrict__ aux) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  const float *e = E + r * lde;
-  uint8_t *o = out + r * (int64_t)(K + 16);
-  double s = 0.0;
-  float amax = 0.f;
-  for (int t = 0; t < D; ++t) {
-    const float x = e[t];
-    s += (double)x * (double)x;
-    amax = fmaxf(amax, fabsf(role == 0 ? x : 2.0f * x));
-  }
-  int ex = 0;
-  if (amax > 0.f) {
-    ex = (int)ceilf(log2f(amax / 448.0f));
-    while (ldexpf(amax, -ex) > 448.0f) ++ex;
-    ex = max(-126, min(126, ex));
-  }
-  for (int t = 0; t < D; ++t) {
-    const float x = role == 0 ? e[t] : -2.0f * e[t];
-    o[t] = f2e4m3(ldexpf(x, -ex));
-  }
-  for (int t = D; t < K; ++t) o[t] = 0;
-  float *tf = reinterpret_cast<float *>(o + K);
-  int32_t *ti = reinterpret_cast<int32_t *>(o + K);
-  tf[0] = role == 0 ? (float)s : 0.f;
-  ti[1] = ex + 127;  // E8M0 biased exponent
-  ti[2] = 0;
-  ti[3] = 0;
-  if (aux) aux[r] = (float)s;
-}
-
 // ---------------------------------------------------------------------------------
-// Packing: one thread per row (rows are short: K <= 136 elements).
-__global__ void k_pack_f32(const float *__restrict__ E, int64_t n, int32_t D, int64_t lde,
-                           int role, int32_t K, float *__restrict__ out, float *__restrict__ aux) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  const float *e = E + r * lde;
-  float *o = out + r * K;
-  double s = 0.0;
-  for (int t = 0; t < D; ++t) {
-    float x = e[t];
-    s += (double)x * (double)x;
-    o[t] = role == 0 ? x : -2.0f * x;
-  }
-  o[D] = role == 0 ? (float)s : 1.0f;
-  for (int t = D + 1; t < K; ++t) o[t] = 0.f;
-  if (aux) aux[r] = (float)s;
+// Packing, `rb` rows per workgroup staged through LDS: the FP32 rows are read coalesced with
+// several loads in flight, one thread per row sums the squared norm in feature order (FP64,
+// the value that the BF16 split needs) and, for FP8, finds the row's scale, and all threads
+// then write the packed rows as consecutive 32-bit words.  With a thread per row throughout,
+// every access touched a line per lane: 1.5M FP8 rows of 100 took 4.4 ms (now 187 us),
+// 1M BF16 rows of 50 313 us (now 105).
+//
+// FP32: [r, ||r||^2, 0...] / [-2q, 1, 0...].  BF16: the norm as an unevaluated sum of three
+// bf16 values (24 significant bits).  FP8: x / 2^e in OCP E4M3 (the converter rounds to
+// nearest even; values are clamped to its +-448) with e the smallest power of two that
+// brings max|x| under 448, and a trailer of the norm and e.
+constexpr int kPackThreads = 256;
+constexpr int kPackRows = 64;  // at most
+
+// Smallest e with |amax| / 2^e <= 448, clamped to the E8M0 range (an infinite amax too).
+__device__ __forceinline__ int fp8_exp(float amax) {
+  if (!(amax > 0.f)) return 0;
+  int ex = (int)fminf(fmaxf(ceilf(log2f(amax / 448.0f)), -126.f), 126.f);
+  while (ex < 126 && ldexpf(amax, -ex) > 448.0f) ++ex;
+  return ex;
 }
 
-// BF16 rows, up to 128 per workgroup staged through LDS (at most 64 KiB): the FP32 rows are
-// read coalesced, each thread packs its own row (the squared norm summed over the row in
-// order, as the FP64 value the three-term split needs), and the packed rows are written
-// back coalesced.
-constexpr int kPackRows = 128;
-__global__ void __launch_bounds__(kPackRows) k_pack_bf16(const float *__restrict__ E, int64_t n,
-                                                        int32_t D, int64_t lde, int role,
-                                                        int32_t K, uint16_t *__restrict__ out,
-                                                        float *__restrict__ aux) {
-  extern __shared__ float pack_lds[];
-  const int RB = blockDim.x;  // rows per workgroup (<= kPackRows)
-  float *sE = pack_lds;                                 // [RB][D]
-  uint16_t *sO = (uint16_t *)(pack_lds + RB * D);       // [RB][K]
-  const int tid = threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.x * RB;
-  const int rows = (int)min<int64_t>(RB, n - r0);
-  for (int e = tid; e < rows * D; e += RB) {
-    const int rr = e / D, t = e % D;
-    sE[e] = E[(r0 + rr) * lde + t];
+template <int DT>
+__global__ void __launch_bounds__(kPackThreads) k_pack(const float *__restrict__ E, int64_t n,
+                                                       int32_t D, int64_t lde, int role,
+                                                       int32_t K, int rb,
+                                                       uint32_t *__restrict__ out,
+                                                       float *__restrict__ aux) {
+  extern __shared__ float pack_lds[];  // [rb][D | 1]
+  __shared__ double s_n2[kPackRows];
+  __shared__ int s_ex[kPackRows];
+  const int tid = threadIdx.x, ld = D | 1;
+  const int64_t r0 = (int64_t)blockIdx.x * rb;
+  const int rows = (int)min<int64_t>(rb, n - r0);
+  const float *src = E + r0 * lde;
+#pragma unroll 4
+  for (int e = tid; e < rows * D; e += kPackThreads) {
+    const int r = e / D, t = e - r * D;
+    pack_lds[r * ld + t] = src[r * lde + t];
   }
   __syncthreads();
   if (tid < rows) {
-    const float *e = sE + tid * D;
-    uint16_t *o = sO + tid * K;
+    const float *x = pack_lds + tid * ld;
     double s = 0.0;
+    float amax = 0.f;
+#pragma unroll 4
     for (int t = 0; t < D; ++t) {
-      float x = e[t];
-      s += (double)x * (double)x;
-      o[t] = role == 0 ? f2bf(x) : f2bf(-2.0f * x);
+      s += (double)x[t] * (double)x[t];
+      if (DT == SH_FP8) amax = fmaxf(amax, fabsf(role == 0 ? x[t] : 2.0f * x[t]));
     }
-    if (role == 0) {
-      // ||r||^2 as an unevaluated sum of three bf16 values (24 significant bits)
-      float hi = bf2f(f2bf((float)s));
-      double r1 = s - (double)hi;
-      float mid = bf2f(f2bf((float)r1));
-      double r2 = r1 - (double)mid;
-      float lo = bf2f(f2bf((float)r2));
-      o[D] = f2bf(hi);
-      o[D + 1] = f2bf(mid);
-      o[D + 2] = f2bf(lo);
-    } else {
-      o[D] = o[D + 1] = o[D + 2] = f2bf(1.0f);
-    }
-    for (int t = D + 3; t < K; ++t) o[t] = 0;
+    s_n2[tid] = s;
+    if (DT == SH_FP8) s_ex[tid] = fp8_exp(amax);
     if (aux) aux[r0 + tid] = (float)s;
   }
   __syncthreads();
-  // K is even: write 32-bit pairs
-  const uint32_t *s32 = (const uint32_t *)sO;
-  uint32_t *o32 = (uint32_t *)(out + r0 * K);
-  for (int e = tid; e < rows * K / 2; e += RB) o32[e] = s32[e];
+  const int words = DT == SH_F32 ? K : DT == SH_BF16 ? K / 2 : K / 4 + 4;  // per row
+  for (int e = tid; e < rows * words; e += kPackThreads) {
+    const int r = e / words, wd = e - r * words;
+    const float *x = pack_lds + r * ld;
+    uint32_t o = 0;
+    if (DT == SH_F32) {
+      o = __float_as_uint(wd < D    ? (role == 0 ? x[wd] : -2.0f * x[wd])
+                          : wd == D ? (role == 0 ? (float)s_n2[r] : 1.0f)
+                                    : 0.f);
+    } else if (DT == SH_BF16) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int t = 2 * wd + u;
+        uint16_t b = 0;
+        if (t < D) {
+          b = f2bf(role == 0 ? x[t] : -2.0f * x[t]);
+        } else if (t < D + 3) {
+          if (role == 0) {
+            const double s = s_n2[r];
+            const float hi = bf2f(f2bf((float)s));
+            const double r1 = s - (double)hi;
+            const float mid = bf2f(f2bf((float)r1));
+            const float lo = bf2f(f2bf((float)(r1 - (double)mid)));
+            b = f2bf(t == D ? hi : t == D + 1 ? mid : lo);
+          } else {
+            b = f2bf(1.0f);
+          }
+        }
+        o |= (uint32_t)b << (16 * u);
+      }
+    } else if (wd < K / 4) {
+      float v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = 4 * wd + u;
+        const float y = t < D ? ldexpf(role == 0 ? x[t] : -2.0f * x[t], -s_ex[r]) : 0.f;
+        v[u] = fminf(fmaxf(y, -448.f), 448.f);
+      }
+      int p = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+      p = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], p, true);
+      o = (uint32_t)p;
+    } else if (wd == K / 4) {
+      o = __float_as_uint(role == 0 ? (float)s_n2[r] : 0.f);
+    } else if (wd == K / 4 + 1) {
+      o = (uint32_t)(s_ex[r] + 127);  // E8M0 biased exponent
+    }
+    out[r0 * words + e] = o;
+  }
 }
+
 
 // A query's starting threshold from the threshold pass: the rank-th smallest of its `m`
 // slot minima (k_bound), one wave per query.  The orderable images are searched bit by bit
 // from the top (count the values at or below a prefix); the low kTauSkip bits are left set,
 // which only raises the threshold.  Fewer than `rank` finite minima leave it open.
 constexpr int kTauSkip = 4;
+// Wave sum with DPP lane moves, the same value in every lane.
+__device__ __forceinline__ int wave_sum_i32(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);   // lane ^ 1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);   // lane ^ 2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x124, 0xF, 0xF, true);  // row_ror:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, true);  // row_ror:8
+  return (__builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16)) +
+         (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
+}
+// How many of a wave's E predicates per lane hold.  LANES: every lane counts its own and one
+// wave sum follows, the shorter chain of a wave that works alone; else a ballot and a scalar
+// popcount each, which take fewer vector instructions where many waves share a SIMD (the
+// thresholds of a million queries 427 against 656 us).
+template <bool LANES, int E, class P>
+__device__ __forceinline__ int wave_count(P pred) {
+  int c = 0;
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    if constexpr (LANES)
+      c += pred(i);
+    else
+      c += __popcll(__builtin_amdgcn_ballot_w64(pred(i)));
+  }
+  if constexpr (LANES) c = wave_sum_i32(c);
+  return c;
+}
+
 template <int EL>
 __global__ void __launch_bounds__(256) k_tau(const float *__restrict__ slot_min, int64_t nq,
                                              int m, int rank, float *__restrict__ tau0,
@@ -190,9 +193,7 @@ __global__ void __launch_bounds__(256) k_tau(const float *__restrict__ slot_min,
   uint32_t prefix = 0;
   for (int bit = 31; bit >= kTauSkip; --bit) {
     const uint32_t t = prefix | ((1u << bit) - 1u);
-    int below = 0;
-#pragma unroll
-    for (int i = 0; i < EL; ++i) below += __popcll(__builtin_amdgcn_ballot_w64(v[i] <= t));
+    const int below = wave_count<(EL >= 8), EL>([&](int i) { return v[i] <= t; });
     if (below < rank) prefix |= 1u << bit;
   }
   const uint32_t t = prefix | ((1u << kTauSkip) - 1u);
@@ -234,19 +235,27 @@ __global__ void __launch_bounds__(256) k_pool_merge(
   const int ns = 2 * S, room = cap / 2;
   uint64_t *kept = merge_lds + w * pool;
   int *off = reinterpret_cast<int *>(merge_lds + 4 * pool) + w * ns;
-  int total = 0;
+  // a lane takes a run of consecutive segments: independent loads, one scan over the lanes
+  const int run = (ns + 63) / 64;
+  int mine = 0;
   bool over = false;
-  for (int b = 0; b < ns; b += 64) {
-    const int c = b + lane < ns ? seg_cnt[p * ns + b + lane] : 0;
+  for (int i = 0; i < run; ++i) {
+    const int sg = lane * run + i;
+    const int c = sg < ns ? seg_cnt[p * ns + sg] : 0;
     over |= c > room;
-    int inc = c;
+    if (sg < ns) off[sg] = mine;
+    mine += c;
+  }
+  int inc = mine;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int up = __shfl_up(inc, o, kWave);
-      if (lane >= o) inc += up;
-    }
-    if (b + lane < ns) off[b + lane] = total + inc - c;
-    total += __shfl(inc, 63, kWave);
+  for (int o = 1; o < 64; o <<= 1) {
+    const int up = __shfl_up(inc, o, kWave);
+    if (lane >= o) inc += up;
+  }
+  const int total = __shfl(inc, 63, kWave);
+  for (int i = 0; i < run; ++i) {
+    const int sg = lane * run + i;
+    if (sg < ns) off[sg] += inc - mine;
   }
   if (fail && (wave_any(over) || total < need)) {
     if (lane == 0) fail[atomicAdd(fail_n, 1)] = fail_base + (int32_t)p;
@@ -286,9 +295,15 @@ __global__ void __launch_bounds__(256) k_pool_merge(
       for (int bit = 31; bit >= 0; --bit) {
         const uint32_t t = prefix | ((1u << bit) - 1u);
         int c = 0;
+        if constexpr (BITS) {  // a large scan: many waves, and groups past m are skipped
 #pragma unroll
-        for (int i = 0; i < E; ++i)
-          if (64 * i < m) c += __popcll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) <= t));
+          for (int i = 0; i < E; ++i)
+            if (64 * i < m)
+              c += __popcll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) <= t));
+        } else {
+          c = wave_count<true, E>(
+              [&](int i) { return (uint32_t)(v[i] >> 32) <= t && i * 64 + lane < m; });
+        }
         if (c < pool) prefix |= 1u << bit;
       }
       t_hi = prefix;
@@ -710,21 +725,20 @@ extern "C" int sh_knn_pack(const float *E, int64_t n, int32_t D, int64_t lde, in
     return SH_EUNSUPPORTED;
   }
   if (n == 0) return SH_OK;
-  dim3 grid(cdiv(n, 256)), block(256);
+  // fewer rows a workgroup where the batch would leave the GPU idle
+  const int rb = n >= 64 * 512 ? kPackRows : n >= 16 * 256 ? 16 : 4;
+  const dim3 grid((uint32_t)cdiv(n, rb)), block(kPackThreads);
+  const size_t lds = (size_t)rb * (D | 1) * sizeof(float);
+#define SH_PACK(DT)                                                                             \
+  hipLaunchKernelGGL(k_pack<DT>, grid, block, lds, (hipStream_t)stream, E, n, D, lde, role, K,  \
+                     rb, (uint32_t *)out, aux_out)
   if (dtype == SH_F32)
-    hipLaunchKernelGGL(k_pack_f32, grid, block, 0, (hipStream_t)stream, E, n, D, lde, role, K,
-                       (float *)out, aux_out);
-  else if (dtype == SH_BF16) {
-    const size_t per_row = D * sizeof(float) + K * sizeof(uint16_t);
-    int rb = kPackRows;
-    while (rb > 1 && (size_t)rb * per_row > 65536) rb /= 2;
-    SH_ARG((size_t)rb * per_row <= 65536, "sh_knn_pack: D=%d too large for the BF16 pack", D);
-    hipLaunchKernelGGL(k_pack_bf16, dim3((uint32_t)cdiv(n, rb)), dim3(rb), (size_t)rb * per_row,
-                       (hipStream_t)stream, E, n, D, lde, role, K, (uint16_t *)out, aux_out);
-  }
+    SH_PACK(SH_F32);
+  else if (dtype == SH_BF16)
+    SH_PACK(SH_BF16);
   else
-    hipLaunchKernelGGL(k_pack_fp8, grid, block, 0, (hipStream_t)stream, E, n, D, lde, role, K,
-                       (uint8_t *)out, aux_out);
+    SH_PACK(SH_FP8);
+#undef SH_PACK
   SH_LAUNCH_CHECK("k_pack");
   return SH_OK;
 }
@@ -873,21 +887,24 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
     p.m = nr >> p.shift;
     const int64_t res1 = (int64_t)std::max(1, ops.bound_resident ? ops.bound_resident(K) : 1) *
                          kCUs;
-    const int max1 = (int)std::min<int64_t>(1024, cdiv(p.m, kSliceAlign));
+    // at most 256 slices here and 512 below: one query's slots and segments are one wave's
+    // work, and past that it takes longer than the slices save
+    const int max1 = (int)std::min<int64_t>(256, cdiv(p.m, kSliceAlign));
     // slots enough that the rank-th smallest minimum is close to the rank-th smallest key
     const int min1 = (int)std::min<int64_t>(max1, cdiv(4 * (int64_t)p.rank, 16));
     const int want1 = (int)std::min<int64_t>(max1, cdiv(res1, qb));
     p.S1 = want1 > min1 ? want1 : pick_slices(qb, res1, min1, std::min(max1, min1 + 4));
     p.len1 = align_up((size_t)cdiv(p.m, p.S1), kSliceAlign);
     p.S1 = (int)cdiv(p.m, p.len1);
-    p.per = 16 * p.S1 <= 2048 ? 8 : 4 * p.S1 <= 2048 ? 2 : 1;
+    p.per = 16 * p.S1 <= 512 ? 8 : 4 * p.S1 <= 512 ? 2 : 1;
+    while (p.per < 8 && p.S1 * 2 * p.per < 4 * p.rank) p.per = p.per == 1 ? 2 : 8;
     p.slots = p.S1 * 2 * p.per;
     int64_t res3;
     if (p.collect) {
       res3 = (int64_t)std::max(1, ops.collect_resident ? ops.collect_resident(K) : 1) * kCUs;
       // a query's keys vary with the sample by 1 / sqrt(rank); all may come from one slice
       const double keys = 1.1 * p.rank * (1 << p.shift);
-      p.cap = (int)align_up((size_t)(keys * (1.0 + 5.5 / std::sqrt((double)p.rank))) + 64, 128);
+      p.cap = (int)align_up((size_t)(keys * (1.0 + 7.5 / std::sqrt((double)p.rank))) + 64, 128);
     } else {
       res3 = (int64_t)std::max(1, ops.screen_resident ? ops.screen_resident(K, p.cap) : 1) *
              kCUs;
@@ -895,7 +912,7 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
     // slices of at least 256 references, at most kBufBytes of candidate buffers
     const int64_t room = std::max<int64_t>(
         1, (int64_t)(kBufBytes / ((size_t)std::max<int64_t>(nq, 1) * p.cap * 8)));
-    const int max3 = (int)std::min<int64_t>(std::min<int64_t>(p.collect ? 256 : 1024, room),
+    const int max3 = (int)std::min<int64_t>(std::min<int64_t>(p.collect ? 256 : 512, room),
                                             std::max<int64_t>(1, nr / 256));
     const int want3 = (int)cdiv(res3, qb);
     p.S3 = want3 >= max3 ? max3
