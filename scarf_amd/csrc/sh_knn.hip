@@ -853,9 +853,16 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
   const KnnOps ops = knn_ops(dtype);
   const int64_t qb = std::max<int64_t>(1, cdiv(nq, 256));
   p.bounded = nr >= 8 * (int64_t)pool;
-  // below about a billion pairs (some 0.1 ms of scan) the launches of the second screen
-  // cost more than k_collect saves over k_screen
-  p.collect = p.bounded && (double)nq * (double)nr >= 1e9;
+  // Measured time of a pair in the scan's loop: 0.1 ps for 64 packed BF16 elements, FP8 half,
+  // FP32 0.75 ps for 56.
+  const double c_pair = dtype == SH_F32    ? 0.75e-12 * K / 56
+                        : dtype == SH_BF16 ? 0.1e-12 * K / 64
+                                           : 0.055e-12 * K / 64;
+  // Below some 5 us of scan the launches of the second screen cost what k_collect saves over
+  // k_screen: whole calls take 61.7 us with k_screen and 63.5 with k_collect at 100 queries x
+  // 100,000 references (BF16, D = 50), 88 and 81 at 1000 x 100,000, 155 and 135 at
+  // 1000 x 500,000, 433 and 353 at 4000 x 500,000.
+  p.collect = p.bounded && (double)nq * (double)nr * c_pair >= 5e-6;
   p.cap = screen_cap(pool);
   p.S1 = p.S3 = 1;
   p.len3 = align_up((size_t)nr, kSliceAlign);
@@ -867,9 +874,6 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
     // meets one in two tiles (the tile leaves the short path for it alone), twice that for
     // FP8.  The million-cell self search takes 174 / 152 / 146 / 146 ms with s = 2 / 4 / 8 /
     // 16, the 100,000-cell one 2.91 / 2.68 / 2.67 / 2.87.
-    const double c_pair = dtype == SH_F32    ? 0.75e-12 * K / 56
-                          : dtype == SH_BF16 ? 0.1e-12 * K / 64
-                                             : 0.055e-12 * K / 64;
     double best = 0.0;
     for (int sh = 0; sh <= 4; ++sh) {
       if (sh > 0 && (nr >> sh) < 8 * (int64_t)pool) break;
