@@ -260,45 +260,141 @@ __global__ void __launch_bounds__(256) k_densify(
 // groups' sums are added in a fixed order at the end of the row.  DPL = 64-column
 // passes (D <= 64 * DPL).
 //
-// The gathers are the traffic (a W row per non-zero, from L2), and what bounds it is the
-// L1's share of them: eight gathers in flight a wave instead of one, rows padded to whole
-// cache lines, and 32-bit row offsets each changed nothing.  A group's own lanes hold its
-// entries (lane i of group g: entry 4 i + g of the batch), so an entry reaches its group by
-// a DPP row broadcast instead of ds_bpermute; the next batch's counts are in flight during
-// this one's gathers.  500,000 x 2000 at 8% non-zeros, D = 50: 1622 -> 1327 us.
+// A group's own lanes hold its entries (lane i of group g: entry 4 i + g of the batch), so an
+// entry reaches its group by a DPP row broadcast, which for W's address is part of the add;
+// the normalised value of a count below 64 comes from lane `count` of a per-row table, since
+// most counts are small and log1pf is 70 instructions; the next batch's counts are in flight
+// during this one's gathers.  Together that took the vector instructions from 477 to 324
+// million at 500,000 x 2000 with 8% non-zeros and D = 50, and the time from 1327 to 1298 us:
+// what bounds it there is the L1's share of the gathers (16.6 GB).  k_project_hot takes them
+// from LDS.
 constexpr int kProjGroup = 16;
 template <int I>
 __device__ __forceinline__ int row_bcast(int v) {  // lane I of each 16-lane row
   return __builtin_amdgcn_update_dpp(0, v, 0x150 + I, 0xF, 0xF, true);
 }
-template <int DPL, int I>
-__device__ __forceinline__ void project_step(int f, float delta, int cnt, int c4,
-                                             const bool (&col_ok)[DPL], const float4 *W4,
-                                             uint32_t ld4, float4 (&acc)[DPL]) {
-  if (4 * I >= cnt) return;  // the same for the whole wave
-  const int fj = row_bcast<I>(f);
-  const float dj = __int_as_float(row_bcast<I>(__float_as_int(delta)));
-  if (fj >= 0) {
+// library size over the mapped columns (the mapping target's), for the whole wave
+__device__ __forceinline__ double mapped_libsize(const uint32_t *vals, const int32_t *cols,
+                                                 int64_t a, int64_t b, const int32_t *col_map,
+                                                 int32_t n_in, int lane) {
+  uint64_t s = 0;
+  for (int64_t t = a + lane; t < b; t += 64)
+    if (map_col(col_map, cols[t], n_in) >= 0) s += vals[t];
+  s = wave_sum_u64(s);
+  return s == 0 ? 1.0 : (double)s;
+}
+// normalised value of a count below 64, lane v's for count v
+__device__ __forceinline__ float project_lut(float scale, int log_t, int lane) {
+  const float x = (float)lane * scale;
+  return log_t ? log1pf(x) : x;
+}
+// an entry's feature (-1: none) and what its W row is multiplied by
+__device__ __forceinline__ float project_delta(uint32_t v, int32_t c, bool there, float lut,
+                                               float scale, int log_t, const int32_t *col_map,
+                                               int32_t n_in, const float *mu,
+                                               const float *inv_sigma, int stride, float clip,
+                                               int *feature) {
+  float xv = __int_as_float(
+      __builtin_amdgcn_ds_bpermute((int)(min(v, 63u) << 2), __float_as_int(lut)));
+  const int f = there ? map_col(col_map, c, n_in) : -1;
+  *feature = f;
+  if (f < 0) return 0.f;
+  if (v > 63u) {
+    const float x = (float)v * scale;
+    xv = log_t ? log1pf(x) : x;
+  }
+  const float is = inv_sigma[f * stride];
+  if (clip > 0.f) {
+    const float m = mu[f * stride];
+    const float zs = (xv - m) * is;
+    const float z0 = (0.f - m) * is;
+    return fminf(fmaxf(zs, -clip), clip) - fminf(fmaxf(z0, -clip), clip);
+  }
+  return xv * is;
+}
+// steps (of four entries) whose loads are all in flight before the first is used
+constexpr int kProjSteps = 8;
+// W's address for a lane: `at` is the entry's byte offset (its row index if WIDE), `lo` the
+// lane's own
+template <bool WIDE>
+__device__ __forceinline__ float4 project_load(int at, uint32_t lo, const char *W,
+                                               int64_t row_bytes) {
+  if (WIDE) return *reinterpret_cast<const float4 *>(W + (int64_t)at * row_bytes + lo);
+  return *reinterpret_cast<const float4 *>(W + ((uint32_t)at + lo));
+}
+template <int DPL>
+__device__ __forceinline__ void project_add(float dj, const float4 (&w)[DPL], float4 (&acc)[DPL]) {
 #pragma unroll
-    for (int p = 0; p < DPL; ++p) {
-      if (col_ok[p]) {
-        const float4 w = W4[(uint64_t)(uint32_t)fj * ld4 + c4 + kProjGroup * p];
-        acc[p].x = fmaf(dj, w.x, acc[p].x);
-        acc[p].y = fmaf(dj, w.y, acc[p].y);
-        acc[p].z = fmaf(dj, w.z, acc[p].z);
-        acc[p].w = fmaf(dj, w.w, acc[p].w);
-      }
+  for (int p = 0; p < DPL; ++p) {
+    acc[p].x = fmaf(dj, w[p].x, acc[p].x);
+    acc[p].y = fmaf(dj, w[p].y, acc[p].y);
+    acc[p].z = fmaf(dj, w[p].z, acc[p].z);
+    acc[p].w = fmaf(dj, w[p].w, acc[p].w);
+  }
+}
+// Entries that are none (behind the row's end, or of a feature that is not taken) are masked,
+// in scalar instructions; a block without any skips that.  0 * 0 is added for them: W itself
+// may hold an infinity.
+template <int DPL, bool WIDE, int B, int... I>
+__device__ __forceinline__ void project_steps(std::integer_sequence<int, I...>, int at,
+                                              float delta, uint64_t valid,
+                                              const uint32_t (&lo)[DPL], const char *W,
+                                              int64_t row_bytes, float4 (&acc)[DPL]) {
+  constexpr uint64_t kStep = 0x0001000100010001ull;  // lane 0 of each group
+  constexpr uint64_t kAll = (((1ull << kProjSteps) - 1) << B) * kStep;
+  float4 w[kProjSteps][DPL];
+  if ((valid & kAll) == kAll) {
+    (
+        [&] {
+#pragma unroll
+          for (int p = 0; p < DPL; ++p)
+            w[I][p] = project_load<WIDE>(row_bcast<B + I>(at), lo[p], W, row_bytes);
+        }(),
+        ...);
+  } else {
+    (
+        [&] {
+          const uint64_t m = (valid >> (B + I)) & kStep;
+#pragma unroll
+          for (int p = 0; p < DPL; ++p) w[I][p] = make_float4(0.f, 0.f, 0.f, 0.f);
+          if (__builtin_amdgcn_inverse_ballot_w64((m << 16) - m)) {
+#pragma unroll
+            for (int p = 0; p < DPL; ++p)
+              w[I][p] = project_load<WIDE>(row_bcast<B + I>(at), lo[p], W, row_bytes);
+          }
+        }(),
+        ...);
+  }
+  (project_add<DPL>(__int_as_float(row_bcast<B + I>(__float_as_int(delta))), w[I], acc), ...);
+}
+// groups 0 + 1 and 2 + 3, then the two pairs
+template <int DPL>
+__device__ __forceinline__ void project_store(float4 (&acc)[DPL], const bool (&col_ok)[DPL],
+                                              int grp, int c4, int32_t D, const float *cvec,
+                                              float *e) {
+  const int lane = grp * kProjGroup + c4;
+  auto from = [](int l, float x) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(l << 2, __float_as_int(x)));
+  };
+  auto add = [&](int l, float4 &x) {
+    x = make_float4(x.x + from(l, x.x), x.y + from(l, x.y), x.z + from(l, x.z),
+                    x.w + from(l, x.w));
+  };
+#pragma unroll
+  for (int p = 0; p < DPL; ++p) {
+    add(lane ^ 16, acc[p]);
+    add(lane ^ 32, acc[p]);
+    const int col = 4 * (c4 + kProjGroup * p);
+    if (grp == 0 && col_ok[p]) {
+      float *o = e + col;
+      o[0] = acc[p].x + cvec[col];
+      if (col + 1 < D) o[1] = acc[p].y + cvec[col + 1];
+      if (col + 2 < D) o[2] = acc[p].z + cvec[col + 2];
+      if (col + 3 < D) o[3] = acc[p].w + cvec[col + 3];
     }
   }
 }
-template <int DPL, int... I>
-__device__ __forceinline__ void project_batch(std::integer_sequence<int, I...>, int f,
-                                              float delta, int cnt, int c4,
-                                              const bool (&col_ok)[DPL], const float4 *W4,
-                                              uint32_t ld4, float4 (&acc)[DPL]) {
-  (project_step<DPL, I>(f, delta, cnt, c4, col_ok, W4, ld4, acc), ...);
-}
-template <int DPL>
+template <int DPL, bool WIDE>
 __global__ void __launch_bounds__(256) k_project(
     const uint32_t *__restrict__ vals, const int32_t *__restrict__ cols,
     const int64_t *__restrict__ rowptr, int64_t n_rows, const int32_t *__restrict__ col_map,
@@ -311,22 +407,20 @@ __global__ void __launch_bounds__(256) k_project(
   if (row >= n_rows) return;
   const int grp = lane / kProjGroup, c4 = lane % kProjGroup;
   const int64_t a = rowptr[row], b = rowptr[row + 1];
-  double l;
-  if (libsize) {
-    l = libsize[row];
-  } else {  // library size over the mapped columns (the mapping target's)
-    uint64_t s = 0;
-    for (int64_t t = a + lane; t < b; t += 64)
-      if (map_col(col_map, cols[t], n_in) >= 0) s += vals[t];
-    s = wave_sum_u64(s);
-    l = s == 0 ? 1.0 : (double)s;
-  }
-  const float scale = sf / (float)l;
-  const uint32_t ld4 = (uint32_t)(ldw / 4);
-  const float4 *W4 = reinterpret_cast<const float4 *>(W);
+  const float scale =
+      sf / (float)(libsize ? libsize[row] : mapped_libsize(vals, cols, a, b, col_map, n_in, lane));
+  const char *Wb = reinterpret_cast<const char *>(W);
+  const int64_t row_bytes = ldw * 4;
+  // lanes past a row's last columns load them again and store nothing
   bool col_ok[DPL];
+  uint32_t lo[DPL];
 #pragma unroll
-  for (int p = 0; p < DPL; ++p) col_ok[p] = 4 * (c4 + kProjGroup * p) < D;
+  for (int p = 0; p < DPL; ++p) {
+    const int c = c4 + kProjGroup * p;
+    col_ok[p] = 4 * c < D;
+    lo[p] = 16u * (uint32_t)min(c, (D - 1) / 4);
+  }
+  const float lut = project_lut(scale, log_t, lane);
   float4 acc[DPL];
 #pragma unroll
   for (int p = 0; p < DPL; ++p) acc[p] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -345,45 +439,278 @@ __global__ void __launch_bounds__(256) k_project(
       cn = cols[tn];
       vn = vals[tn];
     }
-    int f = -1;
-    float delta = 0.f;
-    if (t0 + mine < b) {
-      f = map_col(col_map, c, n_in);
-      if (f >= 0) {
-        const float x = (float)v * scale;
-        const float xv = log_t ? log1pf(x) : x;
-        if (clip > 0.f) {
-          const float zs = (xv - mu[f]) * inv_sigma[f];
-          const float z0 = (0.f - mu[f]) * inv_sigma[f];
-          delta = fminf(fmaxf(zs, -clip), clip) - fminf(fmaxf(z0, -clip), clip);
-        } else {
-          delta = xv * inv_sigma[f];
-        }
-      }
-    }
-    project_batch<DPL>(std::make_integer_sequence<int, kProjGroup>{}, f, delta,
-                       (int)min<int64_t>(64, b - t0), c4, col_ok, W4, ld4, acc);
+    int f;
+    const float delta = project_delta(v, c, t0 + mine < b, lut, scale, log_t, col_map, n_in, mu,
+                                      inv_sigma, 1, clip, &f);
+    const uint64_t valid = __ballot(f >= 0);
+    const int at = WIDE ? f : (int)((uint32_t)f * (uint32_t)row_bytes);
+    const auto seq = std::make_integer_sequence<int, kProjSteps>{};
+    project_steps<DPL, WIDE, 0>(seq, at, delta, valid, lo, Wb, row_bytes, acc);
+    if (b - t0 > 4 * kProjSteps)
+      project_steps<DPL, WIDE, kProjSteps>(seq, at, delta, valid, lo, Wb, row_bytes, acc);
     c = cn;
     v = vn;
   }
-  // groups 0 + 1 and 2 + 3, then the two pairs
+  project_store<DPL>(acc, col_ok, grp, c4, D, cvec, E + row * lde);
+}
+
+// The same projection with the rows of W that are used most in LDS: one workgroup of 16 waves
+// a CU for the whole launch.  Non-zeros are uneven over features (of 2000 features the 700 most
+// used hold about 80% of them), and LDS gives a row twice as fast as L1 and without L2 behind
+// it.  Which rows those are does not change a result, so each workgroup chooses by itself, from
+// the features it counts in kHotSample rows of each wave (2, 8, 16, 32, 64: 984, 990, 1005,
+// 1030, 1078 us against 990 with 4).  LDS also holds mean and 1 / sigma (gathered from L1 they
+// cost 115 us) and each feature's place in the table.  An entry reads the table's row, or its
+// row of zeros, and then, under a mask of the groups that have one, W's row in global memory
+// over it; both halves of a batch are in flight at once, and during them the next batch is
+// normalised.  A wave reads the bounds and scales of 64 rows at once and a row's first batches
+// during the row before, so no row waits for a chain of loads.  The additions and their order
+// are those of k_project.
+//
+// 500,000 x 2000 at 8%, D = 50: 1298 -> 855 us (930 under a profiler).  Without the masked loads it would be about
+// 670, and about 460 without any gather: what is left is shared between the row's own reads,
+// vector instructions (about 0.45 ms of them) and L2 latency of the last 20%.
+constexpr int kHotLds = 158 * 1024;    // of a CU's 160 KB
+constexpr uint16_t kHotNone = 0xffff;  // a feature whose row is not in the table
+constexpr int kHotThreads = 1024;
+constexpr int kHotBlocks = 256;  // one a CU
+constexpr int kHotSample = 4;    // rows a wave samples for the counts
+// Building the table costs 15-70 us a launch, more with more features, so it takes 32 rows a
+// wave to pay: at 131,072 rows 111 us against 108 at 600 features and 8%, 145 / 157 at 1000,
+// 239 / 279 at 2000, 511 / 700 at 4000 (8%) and 527 / 699 at 6000, 746 / 923 at 8000 (5%); at
+// half as many rows 64 / 58, 139 / 148, 261 / 291.  Beyond 8192 features the means and places
+// leave less than half of LDS to the table.
+constexpr int64_t kHotRows = (int64_t)kHotBlocks * (kHotThreads / 64) * 32;
+constexpr int kHotMaxD = 8192;
+
+// explicitly LDS: through a generic pointer the compiler joins the two sources of an entry's
+// row into one flat load
+typedef const __attribute__((address_space(3))) char *LdsBytes;
+__device__ __forceinline__ float4 lds_float4(LdsBytes p, uint32_t at) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const f4 x = *(const __attribute__((address_space(3))) f4 *)(p + at);
+  return make_float4(x.x, x.y, x.z, x.w);
+}
+// an entry of a batch on its lane: what its row is multiplied by, where that is in the table
+// (the row of zeros if nowhere) and in W, in bytes; and the wave's entries not in the table
+struct HotEntry {
+  float delta;
+  int hat, at;
+  uint64_t cold;
+};
+template <int B, int... I>
+__device__ __forceinline__ void hot_gather(std::integer_sequence<int, I...>, const HotEntry &e,
+                                           uint32_t lo, LdsBytes tab, const char *W,
+                                           float4 (&w)[kProjSteps][1]) {
+  constexpr uint64_t kStep = 0x0001000100010001ull;  // lane 0 of each group
+  ((w[I][0] = lds_float4(tab, (uint32_t)row_bcast<B + I>(e.hat) + lo)), ...);
+  (
+      [&] {
+        const uint64_t m = (e.cold >> (B + I)) & kStep;
+        if (__builtin_amdgcn_inverse_ballot_w64((m << 16) - m))
+          w[I][0] = project_load<false>(row_bcast<B + I>(e.at), lo, W, 0);
+      }(),
+      ...);
+}
+template <int B, int... I>
+__device__ __forceinline__ void hot_add(std::integer_sequence<int, I...>, float delta,
+                                        const float4 (&w)[kProjSteps][1], float4 (&acc)[1]) {
+  (project_add<1>(__int_as_float(row_bcast<B + I>(__float_as_int(delta))), w[I], acc), ...);
+}
+constexpr int kProjQueue = 4;  // batches of a row loaded ahead
+struct ProjQueue {
+  int32_t c[kProjQueue];
+  uint32_t v[kProjQueue];
+  // the first batches of a row of n entries
+  __device__ __forceinline__ void load(const uint32_t *vals, const int32_t *cols, int n, int mine) {
 #pragma unroll
-  for (int p = 0; p < DPL; ++p) {
-    acc[p].x += __shfl_xor(acc[p].x, 16, 64);
-    acc[p].y += __shfl_xor(acc[p].y, 16, 64);
-    acc[p].z += __shfl_xor(acc[p].z, 16, 64);
-    acc[p].w += __shfl_xor(acc[p].w, 16, 64);
-    acc[p].x += __shfl_xor(acc[p].x, 32, 64);
-    acc[p].y += __shfl_xor(acc[p].y, 32, 64);
-    acc[p].z += __shfl_xor(acc[p].z, 32, 64);
-    acc[p].w += __shfl_xor(acc[p].w, 32, 64);
-    const int col = 4 * (c4 + kProjGroup * p);
-    if (grp == 0 && col_ok[p]) {
-      float *o = E + row * lde + col;
-      o[0] = acc[p].x + cvec[col];
-      if (col + 1 < D) o[1] = acc[p].y + cvec[col + 1];
-      if (col + 2 < D) o[2] = acc[p].z + cvec[col + 2];
-      if (col + 3 < D) o[3] = acc[p].w + cvec[col + 3];
+    for (int i = 0; i < kProjQueue; ++i) fetch(i, vals, cols, 64 * i, n, mine);
+  }
+  __device__ __forceinline__ void fetch(int i, const uint32_t *vals, const int32_t *cols, int t,
+                                        int n, int mine) {
+    c[i] = -1;
+    v[i] = 0;
+    if (t + mine < n) {
+      c[i] = cols[t + mine];
+      v[i] = vals[t + mine];
+    }
+  }
+  // drop the first batch and load the one that starts at entry t
+  __device__ __forceinline__ void next(const uint32_t *vals, const int32_t *cols, int t, int n,
+                                       int mine) {
+#pragma unroll
+    for (int i = 0; i + 1 < kProjQueue; ++i) {
+      c[i] = c[i + 1];
+      v[i] = v[i + 1];
+    }
+    if (t < n) fetch(kProjQueue - 1, vals, cols, t, n, mine);
+  }
+};
+__device__ __forceinline__ int64_t lane_i64(int64_t x, int i) {
+  return (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)x, i) |
+         ((int64_t)__builtin_amdgcn_readlane((int)(x >> 32), i) << 32);
+}
+template <bool MAPPED>
+__global__ void __launch_bounds__(kHotThreads) k_project_hot(
+    const uint32_t *__restrict__ vals, const int32_t *__restrict__ cols,
+    const int64_t *__restrict__ rowptr, int64_t n_rows, const int32_t *__restrict__ map,
+    int32_t n_in, int32_t d, float sf, int log_t, const double *__restrict__ libsize,
+    const float *__restrict__ mu, const float *__restrict__ inv_sigma, float clip,
+    const float *__restrict__ W, int64_t ldw, int32_t D, const float *__restrict__ cvec,
+    float *__restrict__ E, int64_t lde) {
+  __shared__ float4 mem[kHotLds / 16];
+  const int32_t *col_map = MAPPED ? map : nullptr;
+  constexpr int kWaves = kHotThreads / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int grp = lane / kProjGroup, c4 = lane % kProjGroup;
+  const uint32_t ld4 = (uint32_t)(ldw / 4);
+  const uint32_t td4 = (uint32_t)(D + 3) / 4;  // the table's rows are packed
+  const int slot4 = (d + 7) / 8 + (d + 1) / 2;  // the slots' and (mean, 1 / sigma) pairs' share
+  const int hot = (kHotLds / 16 - 32 - slot4) / (int)td4 - 1;  // and a row of zeros
+  int *red = reinterpret_cast<int *>(mem);  // 2 x 16 wave counts, a cursor
+  uint16_t *slot = reinterpret_cast<uint16_t *>(mem + 32);
+  float2 *mi = reinterpret_cast<float2 *>(mem + 32 + (d + 7) / 8);
+  float4 *tab = mem + 32 + slot4;
+  uint32_t *hist = reinterpret_cast<uint32_t *>(tab);
+  const float4 *W4 = reinterpret_cast<const float4 *>(W);
+  const int64_t rstep = (int64_t)gridDim.x * kWaves;
+  const int64_t row0 = (int64_t)blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(wave);
+
+  // counts over the sample
+  for (int f = tid; f < d; f += kHotThreads) {
+    hist[f] = 0;
+    mi[f] = make_float2(mu[f], inv_sigma[f]);
+  }
+  if (tid == 0) red[32] = 0;
+  __syncthreads();
+  const int64_t mine_rows = row0 < n_rows ? (n_rows - row0 + rstep - 1) / rstep : 0;
+  for (int q = 0; q < kHotSample; ++q) {
+    const int64_t k = mine_rows * q / kHotSample;
+    if (mine_rows > 0) {
+      const int64_t r = row0 + k * rstep;
+      const int64_t a = rowptr[r], b = rowptr[r + 1];
+      for (int64_t t = a + lane; t < b; t += 64) {
+        const int f = map_col(col_map, cols[t], n_in);
+        if (f >= 0 && f < d) atomicAdd(&hist[f], 1u);
+      }
+    }
+  }
+  __syncthreads();
+  // the smallest count that at most `hot` features reach; those of the count below it fill up
+  uint32_t under = 0, least = 1;
+  bool fits = d <= hot;
+  if (!fits) {
+    int par = 0;
+    auto reach = [&](uint32_t T) {
+      int n = 0;
+      for (int f = tid; f < d; f += kHotThreads) n += hist[f] >= T;
+      for (int m = 32; m >= 1; m >>= 1) n += __shfl_xor(n, m, 64);
+      if (lane == 0) red[par * 16 + wave] = n;
+      __syncthreads();
+      n = 0;
+      for (int i = 0; i < kWaves; ++i) n += red[par * 16 + i];
+      par ^= 1;
+      return n;
+    };
+    while (least < 0x40000000u && reach(least) > hot) {
+      under = least;
+      least *= 2;
+    }
+    while (least - under > 1) {
+      const uint32_t mid = under + (least - under) / 2;
+      if (reach(mid) > hot)
+        under = mid;
+      else
+        least = mid;
+    }
+  }
+  __syncthreads();
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int f = tid; f < d; f += kHotThreads) {
+      const uint32_t h = hist[f];
+      if (fits) {
+        if (pass == 0) slot[f] = (uint16_t)(f * td4);
+      } else if (pass == 0 ? h >= least : h == under) {
+        const int q = atomicAdd(&red[32], 1);
+        slot[f] = q < hot ? (uint16_t)(q * (int)td4) : kHotNone;
+      } else if (pass == 0) {
+        slot[f] = kHotNone;
+      }
+    }
+    __syncthreads();
+  }
+  for (int f = wave * 4 + grp; f < d; f += kWaves * 4) {
+    const int q = slot[f];
+    if (q == kHotNone) continue;
+    for (uint32_t c = c4; c < td4; c += kProjGroup) tab[q + c] = W4[(uint64_t)f * ld4 + c];
+  }
+  if (tid < (int)td4) tab[hot * td4 + tid] = make_float4(0.f, 0.f, 0.f, 0.f);
+  __syncthreads();
+
+  const uint32_t zero = (uint32_t)hot * td4;  // the row of zeros
+  const char *Wb = reinterpret_cast<const char *>(W);
+  const LdsBytes tb = (LdsBytes)(reinterpret_cast<const char *>(tab));
+  const bool col_ok[1] = {4 * c4 < D};
+  const uint32_t lo = 16u * (uint32_t)min(c4, (D - 1) / 4);
+  const int mine = 4 * c4 + grp;
+  for (int64_t k0 = 0; k0 < mine_rows; k0 += 64) {
+    // lane i: the bounds and the scale of this wave's row k0 + i
+    int64_t A = 0, B = 0;
+    float S = 0.f;
+    if (k0 + lane < mine_rows) {
+      const int64_t r = row0 + (k0 + lane) * rstep;
+      A = rowptr[r];
+      B = rowptr[r + 1];
+      if (libsize) S = sf / (float)libsize[r];
+    }
+    const int n_here = (int)min<int64_t>(64, mine_rows - k0);
+    ProjQueue q, nq;
+    int64_t a = lane_i64(A, 0);
+    int n = (int)(lane_i64(B, 0) - a);
+    q.load(vals + a, cols + a, n, mine);
+    for (int i = 0; i < n_here; ++i) {
+      const int64_t row = row0 + (k0 + i) * rstep;
+      const int ni = min(i + 1, n_here - 1);
+      const int64_t na = lane_i64(A, ni);
+      const int nn = (int)(lane_i64(B, ni) - na);
+      nq.load(vals + na, cols + na, nn, mine);
+      const float scale =
+          libsize ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(S), i))
+                  : sf / (float)mapped_libsize(vals, cols, a, a + n, col_map, n_in, lane);
+      const float lut = project_lut(scale, log_t, lane);
+      float4 acc[1] = {make_float4(0.f, 0.f, 0.f, 0.f)};
+      auto entry = [&](int t0) {
+        HotEntry e;
+        int f;
+        e.delta = project_delta(q.v[0], q.c[0], t0 + mine < n, lut, scale, log_t, col_map, n_in,
+                                &mi[0].x, &mi[0].y, 2, clip, &f);
+        const uint32_t at_slot = f >= 0 ? slot[f] : zero;
+        e.cold = __ballot(at_slot == kHotNone);
+        e.hat = 16 * (int)(at_slot == kHotNone ? zero : at_slot);
+        e.at = (int)((uint32_t)f * 4u * (uint32_t)ldw);
+        return e;
+      };
+      HotEntry e = entry(0);
+      for (int t0 = 0; t0 < n; t0 += 64) {
+        const auto seq = std::make_integer_sequence<int, kProjSteps>{};
+        float4 w[kProjSteps][1], x[kProjSteps][1];
+        HotEntry en = e;
+        hot_gather<0>(seq, e, lo, tb, Wb, w);
+        if (n - t0 > 4 * kProjSteps)
+          hot_gather<kProjSteps>(seq, e, lo, tb, Wb, x);
+        if (t0 + 64 < n) {
+          q.next(vals + a, cols + a, t0 + 64 * kProjQueue, n, mine);
+          en = entry(t0 + 64);
+        }
+        hot_add<0>(seq, e.delta, w, acc);
+        if (n - t0 > 4 * kProjSteps)
+          hot_add<kProjSteps>(seq, e.delta, x, acc);
+        e = en;
+      }
+      project_store<1>(acc, col_ok, grp, c4, D, cvec, E + row * lde);
+      q = nq;
+      a = na;
+      n = nn;
     }
   }
 }
@@ -528,14 +855,21 @@ extern "C" int sh_project(const uint32_t *vals, const int32_t *cols, const int64
   SH_ARG(ldw % 4 == 0 && ((uintptr_t)W % 16) == 0,
          "sh_project: W rows must be 16-byte aligned (ldw a multiple of 4)");
   dim3 grid(cdiv(n_rows, 4)), block(256);
-  if (D <= 64)
-    hipLaunchKernelGGL(k_project<1>, grid, block, 0, (hipStream_t)stream, vals, cols, rowptr,
-                       n_rows, col_map, n_cols_in, (float)sf, log_transform, libsize, mu,
-                       inv_sigma, clip, W, ldw, D, c, E_out, lde);
-  else
-    hipLaunchKernelGGL(k_project<2>, grid, block, 0, (hipStream_t)stream, vals, cols, rowptr,
-                       n_rows, col_map, n_cols_in, (float)sf, log_transform, libsize, mu,
-                       inv_sigma, clip, W, ldw, D, c, E_out, lde);
+  // byte offsets into W in 32 bits, if it is that small
+  const bool wide = (uint64_t)d * (uint64_t)ldw * 4 > 0xffffffffull;
+  if (D <= 64 && n_rows >= kHotRows && d <= kHotMaxD && !wide) {
+    hipLaunchKernelGGL(col_map ? k_project_hot<true> : k_project_hot<false>, dim3(kHotBlocks),
+                       dim3(kHotThreads), 0, (hipStream_t)stream, vals, cols, rowptr, n_rows,
+                       col_map, n_cols_in, d, (float)sf, log_transform, libsize, mu, inv_sigma,
+                       clip, W, ldw, D, c, E_out, lde);
+    SH_LAUNCH_CHECK("k_project_hot");
+    return SH_OK;
+  }
+  auto kern = D <= 64 ? (wide ? k_project<1, true> : k_project<1, false>)
+                      : (wide ? k_project<2, true> : k_project<2, false>);
+  hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, vals, cols, rowptr, n_rows,
+                     col_map, n_cols_in, (float)sf, log_transform, libsize, mu, inv_sigma, clip, W,
+                     ldw, D, c, E_out, lde);
   SH_LAUNCH_CHECK("k_project");
   return SH_OK;
 }

@@ -75,3 +75,44 @@ def test_project_edges(cuda, D, mapped):
     # of at most 400 products in four chains of 100, plus the constant
     tol = (100 + 60) * 2.0 ** -24 * (6.0 * np.abs(W).sum(0) + 1.0)
     assert np.all(np.abs(E - z @ W) <= tol[None, :])
+
+
+@pytest.mark.parametrize("d_in,D,clip,mapped", [
+    (3, 1, 0.0, False), (40, 64, 3.0, False), (2500, 50, 3.0, True), (2500, 33, 0.0, False),
+    (8192, 64, 3.0, False)])
+def test_project_tables_equal_general_path(cuda, d_in, D, clip, mapped):
+    """From 131,072 rows on, the most used rows of W come from LDS: the same bits as the general
+    kernel gives for pieces of fewer rows, with all of W in the table and with part of it,
+    empty and long rows, counts on both sides of 64 and an infinity in W."""
+    import torch
+
+    from scarf_amd.device import DeviceCSR, col_map_tensor
+    from scarf_amd.normalize import NormParams
+    from scarf_amd.pca import Projector
+    from scarf_amd.synth import CSR
+    say("project tables", d_in, D, clip, mapped)
+    rng = np.random.default_rng(8)
+    n = 131072 + 5
+    ln = np.minimum(np.array([0, 1, 31, 33, 64, 65, 5, 2, 9, 20])[np.arange(n) % 10], d_in)
+    ln[[7, 70_000, n - 1]] = min(d_in, 1000)
+    rp = np.concatenate([[0], np.cumsum(ln)]).astype(np.int64)
+    within = np.arange(rp[-1]) - np.repeat(rp[:-1], ln)
+    # distinct sorted columns of a row, the low ones the more frequent
+    gap = np.maximum(d_in // np.maximum(np.repeat(ln, ln), 1), 1)
+    cols = np.minimum(within * gap + (rng.random(rp[-1]) ** 3 * gap).astype(np.int64), d_in - 1)
+    vals = np.where(rng.random(rp[-1]) < 0.02, rng.integers(60, 5000, rp[-1]),
+                    rng.integers(1, 8, rp[-1])).astype(np.uint32)
+    csr = DeviceCSR.from_host(CSR(vals, cols.astype(np.int32), rp, d_in))
+    keep = np.sort(rng.choice(d_in, d_in // 2, replace=False)) if mapped else np.arange(d_in)
+    d = keep.shape[0]
+    W = rng.standard_normal((d, D))
+    W[d // 2, 0] = np.inf
+    cm, _ = col_map_tensor(d_in, keep if mapped else None)
+    proj = Projector.build(W, rng.uniform(0.1, 1.0, d), rng.uniform(0.5, 2.0, d), clip=clip)
+    proj.c.zero_()  # finite: the infinity of W stays in the rows that use it
+    E = proj.project(csr, NormParams(), col_map=cm)
+    for a in range(0, n, 50_000):
+        m = min(50_000, n - a)
+        part = proj.project(csr, NormParams(), col_map=cm, row_start=a, n_rows=m)
+        assert torch.equal(E[a:a + m].view(torch.int32), part.view(torch.int32))
+    assert bool(torch.isfinite(E[:, 0]).any()) and not bool(torch.isfinite(E[:, 0]).all())
