@@ -11,6 +11,7 @@
 #include <utility>
 
 #include "sh_common.h"
+#include "sh_log1p.h"
 
 namespace sh {
 
@@ -39,6 +40,24 @@ __global__ void __launch_bounds__(256) k_libsize(const uint32_t *__restrict__ va
   if (sub == 0) out[row] = s == 0 ? 1.0 : (double)s;
 }
 
+// norm_value with the row's 1 / l at hand: the quotient is corrected by its remainder, so it
+// is as good as the division (whose 11 instructions, with the library's log1p, were most of
+// the statistics), and the logarithm comes from a table in LDS.  What the correction or the
+// table is not made for (l = 0, an infinity, next to the ends of the exponent's range) goes
+// the general way; inv_l is NaN where 1 / l itself is of no use.
+__device__ __forceinline__ double stats_inverse(double l) {
+  return l >= 1e-280 && l <= 1e280 ? 1.0 / l : __longlong_as_double(0x7ff8000000000000ll);
+}
+__device__ __forceinline__ double stats_value(uint32_t v, double sf, double2 l, int log_t,
+                                              const LogStep *tab) {
+  if (!log_t) return norm_value(v, sf, l.x, 0);
+  const double a = sf * (double)v;
+  double q = a * l.y;
+  q = fma(fma(-q, l.x, a), l.y, q);
+  if (q <= 1e300 && (q >= 1e-280 || v == 0)) return log1p_table(q, tab);
+  return norm_value(v, sf, l.x, 1);
+}
+
 // Per-feature FP64 sums of x and x^2 over a slab of rows, for columns [c0, c0+cb).
 // Slabs never straddle a chunk: slab s covers rows [c*chunk + j*slab_rows, ...) of
 // chunk c = s / spc, j = s % spc, so every chunk of the matrix is done in one launch.
@@ -52,7 +71,10 @@ __global__ void __launch_bounds__(256) k_libsize(const uint32_t *__restrict__ va
 // a double-buffered batch in LDS, and one wave at a time, in turn, adds a finished batch
 // while the others are at the next.  Batches are added in order, one wave's ds_add lanes
 // meet in a fixed order, so the sums are bitwise reproducible.
-// 500,000 x 2000 at 8% non-zeros: 1455 -> 551 us; 5,000 rows: 626 -> 20 us.
+// 500,000 x 2000 at 8% non-zeros: 1455 -> 551 us; 5,000 rows: 626 -> 20 us.  Counters then
+// showed 189 vector instructions for 64 entries, three quarters of the time: the corrected quotient
+// and the table (stats_value) took it to 400 us.  The two LDS f64 adds are 105 us of LDS time
+// (23 clocks a wave instruction at random features, 8 at consecutive ones).
 constexpr int kStatsThreads = 512;
 constexpr int kStatsResident = 3 * 256;   // workgroups that fit the GPU (LDS)
 constexpr int kStatsMinRows = 16, kStatsMaxRows = 384;  // rows per slab
@@ -62,11 +84,13 @@ __global__ void __launch_bounds__(kStatsThreads, 6) k_norm_stats(
     int64_t slab_rows, const int32_t *__restrict__ col_map, int32_t n_in, int32_t d,
     int32_t cb, double sf, int log_t, const double *__restrict__ libsize,
     double *__restrict__ part /* [n_slabs][2][d] */) {
-  extern __shared__ double acc[];  // [2][cb], library sizes [slab_rows]
+  // [2][cb], (library size, 1 / it) [slab_rows]
+  extern __shared__ __attribute__((aligned(16))) double acc[];
+  __shared__ LogStep slog[kLogSteps];
   __shared__ double bx[2][kStatsThreads];
   __shared__ int16_t bf[2][kStatsThreads];  // column within the block, -1: none
   __shared__ int32_t srp[kStatsMaxRows + 1];
-  double *sls = acc + 2 * cb;
+  double2 *sls = reinterpret_cast<double2 *>(acc + 2 * cb);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int32_t c0 = blockIdx.y * cb;
   const int32_t ncol = min(d, c0 + cb) - c0;
@@ -79,7 +103,11 @@ __global__ void __launch_bounds__(kStatsThreads, 6) k_norm_stats(
   for (int i = tid; i < 2 * cb; i += kStatsThreads) acc[i] = 0.0;
   for (int i = tid; i <= nrow; i += kStatsThreads)
     srp[i] = nrow > 0 ? (int32_t)(rowptr[r0 + i] - e0) : 0;
-  for (int i = tid; i < nrow; i += kStatsThreads) sls[i] = libsize[r0 + i];
+  for (int i = tid; i < nrow; i += kStatsThreads) {
+    const double l = libsize[r0 + i];
+    sls[i] = make_double2(l, stats_inverse(l));
+  }
+  if (tid < kLogSteps) slog[tid] = kLogTable[tid];
   __syncthreads();
   const int32_t total = srp[nrow];
   const uint32_t *sv = vals + e0;
@@ -117,7 +145,7 @@ __global__ void __launch_bounds__(kStatsThreads, 6) k_norm_stats(
       while (srp[row + 1] <= e) ++row;
       f = map_col(col_map, c, n_in) - c0;
       if (f >= 0 && f < ncol)
-        x = norm_value(v, sf, sls[row], log_t);
+        x = stats_value(v, sf, sls[row], log_t, slog);
       else
         f = -1;
     }
@@ -467,9 +495,10 @@ __global__ void __launch_bounds__(256) k_project(
 // during the row before, so no row waits for a chain of loads.  The additions and their order
 // are those of k_project.
 //
-// 500,000 x 2000 at 8%, D = 50: 1298 -> 855 us (930 under a profiler).  Without the masked loads it would be about
-// 670, and about 460 without any gather: what is left is shared between the row's own reads,
-// vector instructions (about 0.45 ms of them) and L2 latency of the last 20%.
+// 500,000 x 2000 at 8%, D = 50: 1298 -> 855 us (930 under a profiler).  Without the masked
+// loads it would be about 670, and about 460 without any gather: what is left is shared
+// between the row's own reads, vector instructions (about 0.45 ms of them) and L2 latency of
+// the last 20%.
 constexpr int kHotLds = 158 * 1024;    // of a CU's 160 KB
 constexpr uint16_t kHotNone = 0xffff;  // a feature whose row is not in the table
 constexpr int kHotThreads = 1024;
@@ -784,7 +813,7 @@ extern "C" int sh_norm_stats(const uint32_t *vals, const int32_t *cols, const in
   // matrices take column blocks (the CSR is re-read per block)
   const int32_t cb = d <= 2048 ? d : (int32_t)cdiv(d, cdiv(d, 2048));
   const int n_cb = (int)cdiv(d, cb);
-  const size_t lds = (2 * (size_t)cb + (size_t)plan.slab_rows) * sizeof(double);
+  const size_t lds = (2 * (size_t)cb + 2 * (size_t)plan.slab_rows) * sizeof(double);
   double *part = (double *)workspace;
   hipLaunchKernelGGL(k_norm_stats, dim3((unsigned)(plan.n_chunks * plan.spc), n_cb),
                      dim3(kStatsThreads), lds, st, vals, cols, rowptr, n_rows, chunk,

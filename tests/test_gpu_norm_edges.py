@@ -116,3 +116,32 @@ def test_project_tables_equal_general_path(cuda, d_in, D, clip, mapped):
         part = proj.project(csr, NormParams(), col_map=cm, row_start=a, n_rows=m)
         assert torch.equal(E[a:a + m].view(torch.int32), part.view(torch.int32))
     assert bool(torch.isfinite(E[:, 0]).any()) and not bool(torch.isfinite(E[:, 0]).all())
+
+
+@pytest.mark.parametrize("sf", [1e-6, 1.0, 1000.0, 1e12])
+def test_stats_values_over_the_range(cuda, sf):
+    """One row a chunk, so that a sum is one value: counts over all of uint32 and stored zeros,
+    library sizes from 0 over 1e-300 and 1e300 to infinity, where the quotient's correction and
+    the logarithm's table hand over to the general way."""
+    import torch
+
+    from scarf_amd.device import DeviceCSR
+    from scarf_amd.normalize import NormParams, feature_stats
+    from scarf_amd.synth import CSR
+    say("stats values", sf)
+    rng = np.random.default_rng(12)
+    n, d = 48, 300
+    vals = np.exp(rng.uniform(0, np.log(2.0 ** 32 - 1), n * d)).astype(np.uint32)
+    vals[rng.random(n * d) < 0.05] = 0
+    vals[5::97] = 2 ** 32 - 1
+    lib = np.concatenate([[0.0, np.inf, 1e-300, 1e300, 5e-324, 1e-281, 1e281],
+                          np.exp(rng.uniform(-20, 40, n - 7))])
+    h = CSR(vals, np.tile(np.arange(d, dtype=np.int32), n), np.arange(n + 1, dtype=np.int64) * d, d)
+    st = feature_stats(DeviceCSR.from_host(h), 1, NormParams(size_factor=sf,
+                                                            renormalize_subset=False),
+                       n_counts=torch.from_numpy(lib))
+    with np.errstate(all="ignore"):
+        x = np.log1p(sf * vals.reshape(n, d).astype(np.float64) / lib[:, None])
+    # the quotient within half a unit in the last place, of which a logarithm passes on at most
+    # as much, and the logarithm within one, on both sides: 3 units, each at most 2^-52
+    np.testing.assert_allclose(st.chunk_sums.cpu().numpy(), x, rtol=3 * 2.0 ** -52, atol=0)
