@@ -382,9 +382,90 @@ __device__ __forceinline__ double sqdist_exact(const float *__restrict__ q_lds,
   return acc;
 }
 
+// sqdist_exact of one row per lane, for a wave: lane i < n has row j (any valid one elsewhere).
+// A lane reading its own row touches 64 rows an instruction, 25 times over at D = 50, and 64
+// rows a wave are more than L1 holds between two of them.  So the wave loads rows together,
+// 128 bytes of eight rows an instruction (16 bytes a lane, on rows aligned to 4), through LDS,
+// with the next 32 features in flight while these are added, in the same order.  36 floats a
+// row: sixteen lanes' 16-byte reads meet no bank twice.
+constexpr int kRankFeat = 32, kRankRow = kRankFeat + 4;
+struct __attribute__((packed, aligned(4))) RankPiece {
+  float x[4];
+};
+__device__ __forceinline__ double sqdist_rows(const float *q_lds, const float *__restrict__ R,
+                                              int64_t ldr, int D, uint32_t j, int n,
+                                              float *tile) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63, sub = lane & 7, r8 = lane >> 3;
+  const float *row[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    row[u] = R + (int64_t)(uint32_t)__shfl((int)j, 8 * u + r8, kWave) * ldr;
+  RankPiece w[8];
+  auto load = [&](int t0) {
+    const int f = t0 + 4 * sub;
+    if (f + 4 <= D) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (8 * u < n) w[u] = *reinterpret_cast<const RankPiece *>(row[u] + f);
+    } else if (f < D) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (8 * u < n) {
+          w[u].x[0] = row[u][f];
+          if (f + 1 < D) w[u].x[1] = row[u][f + 1];
+          if (f + 2 < D) w[u].x[2] = row[u][f + 2];
+        }
+    }
+  };
+  load(0);
+  double acc = 0.0;
+  for (int t0 = 0; t0 < D; t0 += kRankFeat) {
+    if (t0 + 4 * sub < D) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (8 * u < n)
+          *reinterpret_cast<float4 *>(tile + (8 * u + r8) * kRankRow + 4 * sub) =
+              make_float4(w[u].x[0], w[u].x[1], w[u].x[2], w[u].x[3]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (t0 + kRankFeat < D) load(t0 + kRankFeat);
+    const int here = min(kRankFeat, D - t0);
+    const float *mine = tile + lane * kRankRow;
+    auto add = [&](float a, float b) {
+      const double df = (double)a - (double)b;
+      const double sq = df * df;
+      acc = acc + sq;
+    };
+    int t = 0;
+#pragma unroll 4
+    for (; t + 4 <= here; t += 4) {
+      const float4 a = *reinterpret_cast<const float4 *>(q_lds + t0 + t);
+      const float4 b = *reinterpret_cast<const float4 *>(mine + t);
+      add(a.x, b.x);
+      add(a.y, b.y);
+      add(a.z, b.z);
+      add(a.w, b.w);
+    }
+    for (; t < here; ++t) add(q_lds[t0 + t], mine[t]);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  return acc;
+}
+
 // One wave per query: merge the slices' pools to the global best `pool` by screened
 // key, re-rank them exactly, take the best k (+1 with self repair).
-template <int PE>  // pool elements per lane (pool <= 64 * PE)
+// Consecutive queries share candidates and an L2: the grid is a multiple of the eight XCDs, which
+// take workgroups in turn, and each XCD gets a contiguous eighth of the queries.
+// Rows in turn through LDS from here on (us of the kernel with a row a lane / through LDS, D = 50,
+// pool 64): 1 query 7.3 / 7.1 of 500,000 references and 5.4 / 6.2 of 20,000, 256 queries 8.1 /
+// 7.8 and 6.4 / 7.4, 1000 9.2 / 9.2 and 8.6 / 8.5, 2000 13.4 / 12.8 and 11.9 / 10.9, 16,000
+// 71 / 48 and 45 / 39.  Whole searches: 1,000,000 cells 3.61 -> 2.93 ms of rerank, 1,500,000
+// with pools of 128 22.3 -> 13.8; 16 features at a time give 2.65 and 15.7.
+constexpr int64_t kRankRowsFrom = 1024;
+template <int PE, bool ROWS>  // pool elements per lane (pool <= 64 * PE), sqdist_rows
 __global__ void __launch_bounds__(256) k_rerank(
     const float *__restrict__ Q, int64_t nq, int64_t ldq, const float *__restrict__ R,
     int64_t nr, int64_t ldr, int32_t D, const uint64_t *__restrict__ cand,
@@ -392,9 +473,10 @@ __global__ void __launch_bounds__(256) k_rerank(
     const int64_t *__restrict__ self_idx,
     double err_coef, float r_norm_max, double margin, int64_t *__restrict__ idx_out,
     float *__restrict__ dist_out, int32_t *__restrict__ flags) {
-  __shared__ float qv[4][256];
+  __shared__ __attribute__((aligned(16))) float qv[4][256], tile[ROWS ? 4 : 1][64 * kRankRow];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t q = (int64_t)blockIdx.x * 4 + w;
+  const int64_t block = (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  const int64_t q = block * 4 + w;
   if (q >= nq) return;
   float *ql = qv[w];
   for (int t = lane; t < D; t += 64) ql[t] = Q[q * ldq + t];
@@ -458,9 +540,14 @@ __global__ void __launch_bounds__(256) k_rerank(
 #pragma unroll
   for (int i = 0; i < PE; ++i) {
     const int e = lane * PE + i;
+    const uint32_t j = (uint32_t)v[i];
+    double dist = 0.0;
+    if (ROWS && i < npool) {
+      const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)j);
+      dist = sqdist_rows(ql, R, ldr, D, e < npool ? j : first, (npool - i + PE - 1) / PE, tile[w]);
+    }
     if (e < npool) {
-      const uint32_t j = (uint32_t)(v[i] & 0xffffffffu);
-      c[i].d = sqdist_exact(ql, R + (int64_t)j * ldr, D);
+      c[i].d = ROWS ? dist : sqdist_exact(ql, R + (int64_t)j * ldr, D);
       c[i].i = j;
       if (margin > 0.0)
         emax = fmax(emax, fabs((double)ord_float((uint32_t)(v[i] >> 32)) + qn - c[i].d));
@@ -1119,19 +1206,14 @@ extern "C" int sh_knn_rerank(const float *Q, int64_t nq, int64_t ldq, const floa
          pool);
   SH_ARG(Q && R && cand_keys && cand_cnt && idx_out && dist_out, "sh_knn_rerank: NULL pointer");
   if (nq == 0) return SH_OK;
-  dim3 grid(cdiv(nq, 4)), block(256);
-  if (pool <= 64)
-    hipLaunchKernelGGL(k_rerank<1>, grid, block, 0, (hipStream_t)stream, Q, nq, ldq, R, nr, ldr,
-                       D, cand_keys, cand_cnt, pool, n_slices, k, self_offset, self_idx, err_coef,
-                       r_norm_max, margin, idx_out, dist_out, flags_out);
-  else if (pool <= 128)
-    hipLaunchKernelGGL(k_rerank<2>, grid, block, 0, (hipStream_t)stream, Q, nq, ldq, R, nr, ldr,
-                       D, cand_keys, cand_cnt, pool, n_slices, k, self_offset, self_idx, err_coef,
-                       r_norm_max, margin, idx_out, dist_out, flags_out);
-  else
-    hipLaunchKernelGGL(k_rerank<4>, grid, block, 0, (hipStream_t)stream, Q, nq, ldq, R, nr, ldr,
-                       D, cand_keys, cand_cnt, pool, n_slices, k, self_offset, self_idx, err_coef,
-                       r_norm_max, margin, idx_out, dist_out, flags_out);
+  const bool rows = nq >= kRankRowsFrom;
+  auto kern = pool <= 64    ? (rows ? k_rerank<1, true> : k_rerank<1, false>)
+              : pool <= 128 ? (rows ? k_rerank<2, true> : k_rerank<2, false>)
+                            : (rows ? k_rerank<4, true> : k_rerank<4, false>);
+  hipLaunchKernelGGL(kern, dim3((uint32_t)(8 * cdiv(cdiv(nq, 4), 8))), dim3(256), 0,
+                     (hipStream_t)stream, Q, nq, ldq, R, nr, ldr, D, cand_keys, cand_cnt, pool,
+                     n_slices, k, self_offset, self_idx, err_coef, r_norm_max, margin, idx_out,
+                     dist_out, flags_out);
   SH_LAUNCH_CHECK("k_rerank");
   return SH_OK;
 }

@@ -103,3 +103,52 @@ def test_misleading_sample(cuda, shift):
     Q = _rows(nq, D, 11)
     Q[100:5000] = 40.0 + 0.01 * rng.standard_normal((4900, D))
     _compare(torch.from_numpy(Q.astype(np.float32)).cuda(), torch.from_numpy(E).cuda(), "bf16", 64)
+
+
+@pytest.mark.parametrize("D,pool,extra", [(1, 5, 0), (4, 64, 1), (31, 64, 2), (33, 100, 0),
+                                          (50, 64, 0), (64, 128, 3), (65, 200, 1), (256, 256, 0)])
+def test_rerank_of_many_queries_equals_few(cuda, D, pool, extra):
+    """From 1024 queries on the candidates' rows go through LDS: the same bits as for pieces of
+    fewer queries, over feature counts around the 32 of a piece, rows and buffers that are
+    aligned to 4 bytes only, a last row that ends the buffer, and pools from empty to full."""
+    import torch
+    from scarf_amd import _lib
+    from scarf_amd.device import ptr, stream_handle
+    say("rerank", D, pool, extra)
+    rng = np.random.default_rng(21)
+    nq, nr, ld = 1029, 900, D + extra
+    k = min(11, pool)
+    buf = torch.from_numpy(rng.standard_normal(nr * ld + 1).astype(np.float32)).cuda()
+    R = buf[1:1 + nr * ld]
+    Q = torch.from_numpy(rng.standard_normal((nq, D)).astype(np.float32)).cuda()
+    cnt = rng.integers(0, pool + 1, nq).astype(np.int32)
+    cnt[:4] = [0, 1, pool, pool - 1]
+    idx = np.argsort(rng.random((nq, nr)), axis=1)[:, :pool].astype(np.int64)
+    idx[2, 0] = nr - 1
+    key = (np.arange(pool, dtype=np.int64)[None, :] + 0x40000000) << 32  # ascending, positive
+    cand = torch.from_numpy(key | idx).cuda()
+    cnt = torch.from_numpy(cnt).cuda()
+
+    def rank(a, b):
+        oi = torch.full((b - a, k), -7, dtype=torch.int64, device="cuda")
+        od = torch.full((b - a, k), -7.0, device="cuda")
+        fl = torch.full((b - a,), -7, dtype=torch.int32, device="cuda")
+        _lib.call("sh_knn_rerank", ptr(Q[a:b]), b - a, D, ptr(R), nr, ld, D, ptr(cand[a:b]),
+                  ptr(cnt[a:b]), pool, 1, k, -1, None, -1.0, 0.0, 0.0, ptr(oi), ptr(od), ptr(fl),
+                  stream_handle())
+        return oi, od, fl
+
+    whole = rank(0, nq)
+    for a in range(0, nq, 343):
+        for x, y in zip(whole, rank(a, a + 343)):
+            assert torch.equal(x[a:a + 343], y)
+    # and the oracle's: FP64 terms added in feature order
+    i = 2
+    r = R.cpu().numpy().reshape(nr, ld)[:, :D].astype(np.float64)
+    df = Q[i].cpu().numpy().astype(np.float64) - r[idx[i]]
+    d = np.zeros(pool)
+    for t in range(D):
+        d += df[:, t] ** 2
+    order = np.lexsort((idx[i], d))[:k]
+    assert np.array_equal(whole[0][i].cpu().numpy(), idx[i][order])
+    assert np.array_equal(whole[1][i].cpu().numpy(), d[order].astype(np.float32))
