@@ -24,10 +24,10 @@ if ROOT not in sys.path:
 
 METRIC = "cells/s norm+PCA+kNN @1M cells, recall@11 vs FP64 oracle; mapping p50/p99 ms"
 PEAK = {"bf16": 2.5e15, "fp32": 157.3e12, "fp8": 5.0e15, "fp64": 78.6e12}
-# HBM bytes per screen launch from FETCH_SIZE / WRITE_SIZE counter passes scaled by a 1 GiB
-# copy (profiles/screen_bf16_1m_traffic.md, profiles/screen_fp8_4m_traffic.md), keyed by
-# (workload, screen, pool)
-SCREEN_TRAFFIC = {("1m", "bf16", 64): 5.04e11, ("4m", "fp8", 128): 8.64e12}
+# HBM bytes per candidate search (sh_knn_pool) from FETCH_SIZE / WRITE_SIZE counter passes
+# scaled by a 1 GiB copy (profiles/screen_bf16_1m_traffic.md, profiles/screen_fp8_4m_traffic.md),
+# keyed by (workload, screen, pool); the FP8 value holds both passes
+SCREEN_TRAFFIC = {("1m", "bf16", 64): 3.40e11, ("4m", "fp8", 128): 3.00e12}
 
 WORKLOADS = {
     # cells, genes, groups, density, chunk, dims, k, screen, pool, pca mode, recall queries
@@ -427,9 +427,9 @@ def main():
     ms_per_step = 1e3 * elapsed / args.steps
     value = n * args.steps / elapsed
 
-    # dominant kernel: the MFMA kNN screen over every query (algorithmic flops
-    # 2 * nq * nr * D); the FP8 screen's second pass over the flagged queries is a smaller
-    # launch of another instantiation, reported beside it
+    # dominant kernel: the MFMA scan over every query (algorithmic flops 2 * nq * nr * D),
+    # timed with the threshold pass before it and the merge after it; the FP8 screen's second
+    # pass over the flagged queries is a smaller search of its own, reported beside it
     scr = timings.get("screen", [])
     scr_flops = max((f for _, _, f, _ in scr), default=0.0)
     main = [a.elapsed_time(b) for a, b, f, _ in scr if f == scr_flops]
@@ -440,9 +440,8 @@ def main():
     peak = PEAK[wl["screen"]]
     K = {"bf16": 64, "fp32": 56, "fp8": 64}[wl["screen"]] if wl["dims"] <= 50 else \
         {"bf16": 112, "fp32": 104, "fp8": 128}[wl["screen"]]
-    cap = 256 if wl["pool"] <= 64 else 512
     op = {"bf16": "OpBF16", "fp32": "OpF32", "fp8": "OpFP8"}[wl["screen"]]
-    roofline = {"kernel": f"k_screen<{op},{K},{cap}>", "bound": "mfma",
+    roofline = {"kernel": f"k_collect<{op},{K}>", "bound": "mfma",
                 "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                 "frac": achieved / peak,
                 "traffic": SCREEN_TRAFFIC.get((args.workload, wl["screen"], wl["pool"])),

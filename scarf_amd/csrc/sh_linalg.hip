@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(256) k_dgemm_tall(int64_t m, int32_t n, int32_
 //
 // 64 x 64 entries per workgroup, 4 x 4 per thread, the two 64-column strips of Vt in LDS
 // kMmC rows at a time: one thread per entry re-read both strips for every entry (166 us at
-// d = 2000, 51 components; now about 30).
+// d = 2000, 51 components; now 43).
 constexpr int kMmT = 64, kMmC = 32;
 __global__ void __launch_bounds__(256) k_merge_matrix(
     const double *__restrict__ G, int32_t d, double n, const double *__restrict__ bm,
