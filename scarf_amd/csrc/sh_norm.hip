@@ -74,7 +74,11 @@ __device__ __forceinline__ double stats_value(uint32_t v, double sf, double2 l, 
 // 500,000 x 2000 at 8% non-zeros: 1455 -> 551 us; 5,000 rows: 626 -> 20 us.  Counters then
 // showed 189 vector instructions for 64 entries, three quarters of the time: the corrected quotient
 // and the table (stats_value) took it to 400 us.  The two LDS f64 adds are 105 us of LDS time
-// (23 clocks a wave instruction at random features, 8 at consecutive ones).
+// (23 clocks a wave instruction at random features, 8 at consecutive ones).  The batches wait
+// for the wave that adds, so it reads its eight pieces before the first add: 356 us (two waves,
+// one for the squares: 380, they read twice); a thread keeps its row's end in a register: 347.
+// Library sizes summed in here instead of by k_libsize: 601 against 400 + 195, since all
+// workgroups are in that phase at the same time.
 constexpr int kStatsThreads = 512;
 constexpr int kStatsResident = 3 * 256;   // workgroups that fit the GPU (LDS)
 constexpr int kStatsMinRows = 16, kStatsMaxRows = 384;  // rows per slab
@@ -113,16 +117,23 @@ __global__ void __launch_bounds__(kStatsThreads, 6) k_norm_stats(
   const uint32_t *sv = vals + e0;
   const int32_t *sc = cols + e0;
   auto add = [&](int b) {
-    for (int g = 0; g < kStatsThreads; g += 64) {
-      const int f = bf[b][g + lane];
-      const double x = bx[b][g + lane];
-      if (f >= 0) {
-        atomicAdd(&acc[f], x);
-        atomicAdd(&acc[cb + f], x * x);
+    int f[kStatsThreads / 64];
+    double x[kStatsThreads / 64];
+#pragma unroll
+    for (int g = 0; g < kStatsThreads / 64; ++g) {
+      f[g] = bf[b][64 * g + lane];
+      x[g] = bx[b][64 * g + lane];
+    }
+#pragma unroll
+    for (int g = 0; g < kStatsThreads / 64; ++g) {
+      if (f[g] >= 0) {
+        atomicAdd(&acc[f[g]], x[g]);
+        atomicAdd(&acc[cb + f[g]], x[g] * x[g]);
       }
     }
   };
   int row = 0;  // slab-relative row of this thread's current entry
+  int32_t row_end = nrow > 0 ? srp[1] : 0;
   uint32_t v = 0;
   int32_t c = -1;
   if (tid < total) {
@@ -142,7 +153,7 @@ __global__ void __launch_bounds__(kStatsThreads, 6) k_norm_stats(
     int f = -1;
     double x = 0.0;
     if (e < total) {
-      while (srp[row + 1] <= e) ++row;
+      while (row_end <= e) row_end = srp[++row + 1];
       f = map_col(col_map, c, n_in) - c0;
       if (f >= 0 && f < ncol)
         x = stats_value(v, sf, sls[row], log_t, slog);
