@@ -158,6 +158,16 @@ __device__ __forceinline__ int wave_sum_i32(int v) {
   return (__builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16)) +
          (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
 }
+// Wave or, likewise.
+__device__ __forceinline__ uint32_t wave_or_u32(uint32_t x) {
+  int v = (int)x;
+  v |= __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x124, 0xF, 0xF, true);
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, true);
+  return (uint32_t)((__builtin_amdgcn_readlane(v, 0) | __builtin_amdgcn_readlane(v, 16)) |
+                    (__builtin_amdgcn_readlane(v, 32) | __builtin_amdgcn_readlane(v, 48)));
+}
 // How many of a wave's E predicates per lane hold.  LANES: every lane counts its own and one
 // wave sum follows, the shorter chain of a wave that works alone; else a ballot and a scalar
 // popcount each, which take fewer vector instructions where many waves share a SIMD (the
@@ -214,7 +224,10 @@ __global__ void __launch_bounds__(256) k_tau(const float *__restrict__ slot_min,
 // query has fewer): the pool-th smallest is searched bit by bit on the keys' distance half
 // (count what lies at or below a prefix; on the index half too where distances tie), the
 // keys up to it are packed together in LDS, and only they are sorted: at a million queries
-// of about 240 keys, half the time of sorting them all.
+// of about 240 keys, half the time of sorting them all.  The search starts below the bits that
+// all keys share and ends once a count is the pool, some ten rounds instead of 32: 2.41 ->
+// 1.75 ms at a million queries, 228 -> 168 us at 100,000, 14.6 -> 11.8 for one.  (The same in
+// k_tau, whose values end alike less often, took 536 us instead of 426 at a million.)
 //
 // BITS: the segments hold plain float bits above the index (k_collect), not make_key's word.
 // fail (or NULL): queries whose keys are incomplete -- a segment that overflowed, or fewer
@@ -291,8 +304,16 @@ __global__ void __launch_bounds__(256) k_pool_merge(
     next += fresh;
     uint32_t t_hi = 0xffffffffu, t_lo = 0xffffffffu;  // the last key to keep
     if (m > pool) {
-      uint32_t prefix = 0;
-      for (int bit = 31; bit >= 0; --bit) {
+      // from the highest bit in which two keys differ
+      const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)(v[0] >> 32));
+      uint32_t diff = 0;
+#pragma unroll
+      for (int i = 0; i < E; ++i)
+        if (i * 64 + lane < m) diff |= (uint32_t)(v[i] >> 32) ^ first;
+      int bit = 31 - __clz((int)wave_or_u32(diff));
+      uint32_t prefix = bit < 31 ? first >> (bit + 1) << (bit + 1) : 0;
+      bool cut = false;  // exactly `pool` keys lie at or below prefix
+      for (; bit >= 0 && !cut; --bit) {
         const uint32_t t = prefix | ((1u << bit) - 1u);
         int c = 0;
         if constexpr (BITS) {  // a large scan: many waves, and groups past m are skipped
@@ -304,13 +325,14 @@ __global__ void __launch_bounds__(256) k_pool_merge(
           c = wave_count<true, E>(
               [&](int i) { return (uint32_t)(v[i] >> 32) <= t && i * 64 + lane < m; });
         }
-        if (c < pool) prefix |= 1u << bit;
+        cut = c == pool;
+        prefix = cut ? t : c < pool ? prefix | (1u << bit) : prefix;
       }
       t_hi = prefix;
       int below = 0, upto = 0;
 #pragma unroll
       for (int i = 0; i < E; ++i)
-        if (64 * i < m) {
+        if (64 * i < m && !cut) {
           below += __popcll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) < t_hi));
           upto += __popcll(__builtin_amdgcn_ballot_w64((uint32_t)(v[i] >> 32) <= t_hi));
         }
