@@ -254,6 +254,7 @@ size_t sh_knn_screen_workspace(int64_t nq, int32_t pool, int32_t n_slices);
 int sh_knn_pool(const void *qpack, int64_t nq, const void *rpack, int64_t nr, int32_t D,
                 int dtype, int32_t pool, uint64_t *cand_keys, int32_t *cand_cnt,
                 void *workspace, size_t workspace_bytes, sh_stream_t stream);
+/* 0 for what sh_knn_pool refuses. */
 size_t sh_knn_pool_workspace(int64_t nq, int64_t nr, int32_t D, int dtype, int32_t pool);
 /* Self queries: query q is reference self_idx[q] (self_idx non-NULL) or
  * self_offset + q (self_offset >= 0); k + 1 neighbours are ranked and the query's

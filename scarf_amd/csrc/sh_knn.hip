@@ -998,8 +998,7 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
       }
     }
     p.m = nr >> p.shift;
-    const int64_t res1 = (int64_t)std::max(1, ops.bound_resident ? ops.bound_resident(K) : 1) *
-                         kCUs;
+    const int64_t res1 = (int64_t)ops.bound_resident(K) * kCUs;
     // at most 256 slices here and 512 below: one query's slots and segments are one wave's
     // work, and past that it takes longer than the slices save
     const int max1 = (int)std::min<int64_t>(256, cdiv(p.m, kSliceAlign));
@@ -1014,13 +1013,12 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
     p.slots = p.S1 * 2 * p.per;
     int64_t res3;
     if (p.collect) {
-      res3 = (int64_t)std::max(1, ops.collect_resident ? ops.collect_resident(K) : 1) * kCUs;
+      res3 = (int64_t)ops.collect_resident(K) * kCUs;
       // a query's keys vary with the sample by 1 / sqrt(rank); all may come from one slice
       const double keys = 1.1 * p.rank * (1 << p.shift);
       p.cap = (int)align_up((size_t)(keys * (1.0 + 7.5 / std::sqrt((double)p.rank))) + 64, 128);
     } else {
-      res3 = (int64_t)std::max(1, ops.screen_resident ? ops.screen_resident(K, p.cap) : 1) *
-             kCUs;
+      res3 = (int64_t)ops.screen_resident(K, p.cap) * kCUs;
     }
     // slices of at least 256 references, at most kBufBytes of candidate buffers
     const int64_t room = std::max<int64_t>(
@@ -1064,6 +1062,14 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
   return p;
 }
 
+// Whether the kernels that sh_knn_pool launches exist for this packed width.  pool_plan counts
+// on it: it divides by the number of resident workgroups.
+static bool pool_built(int dtype, int32_t D) {
+  const KnnOps ops = knn_ops(dtype);
+  const int32_t K = pack_k(dtype, D);
+  return ops.bound && K > 0 && ops.bound_resident(K) > 0 && ops.collect_resident(K) > 0;
+}
+
 struct MergeArgs {
   const uint64_t *buf;
   const int32_t *seg_cnt;
@@ -1096,9 +1102,9 @@ static void launch_merge(const MergeArgs &a, hipStream_t st) {
 
 extern "C" size_t sh_knn_pool_workspace(int64_t nq, int64_t nr, int32_t D, int dtype,
                                         int32_t pool) {
-  if (nq <= 0 || nr <= 0 || D <= 0 || pool < 1 || pool > 256) return 0;
-  const int32_t K = pack_k(dtype, D);
-  return K > 0 ? pool_plan(nq, nr, K, dtype, pool).bytes : 0;
+  if (nq <= 0 || nq > 0x7fffffffll || nr <= 0 || nr >= 0xffffffffll || D <= 0) return 0;
+  if (pool < 1 || pool > (dtype == SH_FP8 ? 256 : 128) || !pool_built(dtype, D)) return 0;
+  return pool_plan(nq, nr, pack_k(dtype, D), dtype, pool).bytes;
 }
 
 extern "C" int sh_knn_pool(const void *qpack, int64_t nq, const void *rpack, int64_t nr,
@@ -1115,7 +1121,7 @@ extern "C" int sh_knn_pool(const void *qpack, int64_t nq, const void *rpack, int
   SH_ARG(qpack && rpack && cand_keys && cand_cnt, "sh_knn_pool: NULL pointer");
   const int32_t K = pack_k(dtype, D);
   const KnnOps ops = knn_ops(dtype);
-  if (!ops.bound || K <= 0 || !ops.bound_resident(K)) {
+  if (!pool_built(dtype, D)) {
     set_error("sh_knn_pool: dtype %d with packed K=%d not supported", dtype, K);
     return SH_EUNSUPPORTED;
   }

@@ -1,0 +1,54 @@
+"""CPU-only: how sh_knn_pool plans a search.  A width or size that is not built is an error of
+the call, as for sh_knn_screen, whatever the size of the search."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from scarf_amd import _lib
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+# packed widths that sh_knn_{bf16,fp8,f32}.hip build
+WIDTHS = {"SH_BF16": {16 * i for i in range(1, 9)}, "SH_FP8": {64, 128},
+          "SH_F32": {8 * i for i in range(1, 18)}}
+
+# in a process of its own: an arithmetic trap must not take the test run with it
+SWEEP = """
+from scarf_amd import _lib
+L = _lib.lib()
+for name in ("SH_BF16", "SH_FP8", "SH_F32"):
+    code = getattr(_lib, name)
+    for D in range(1, 257):
+        for nq, nr in ((1, 1), (1, 500_000), (4700, 4700), (10_000, 10_000), (16_384, 500_000),
+                       (1_000_000, 1_000_000), (1 << 53, 1_000_000), (1000, 1 << 40)):
+            for pool in (1, 64, 128, 256):
+                ws = L.sh_knn_pool_workspace(nq, nr, D, code, pool)
+                print(name, L.sh_knn_pack_k(code, D), nq, nr, pool, ws)
+print(L.sh_knn_pool_workspace(10, 10, 8, 77, 64))
+"""
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="libscarfhip.so not built")
+def test_workspace_of_every_width():
+    r = subprocess.run([sys.executable, "-c", SWEEP], cwd=ROOT, capture_output=True, text=True)
+    assert r.returncode == 0, f"exit status {r.returncode}: {r.stderr[-500:]}"
+    *lines, unknown = r.stdout.splitlines()
+    assert unknown == "0"
+    for line in lines:
+        name, K, nq, nr, pool, ws = line.split()
+        built = int(K) in WIDTHS[name] and (int(pool) <= 128 or name == "SH_FP8")
+        fits = int(nq) < 1 << 31 and int(nr) < (1 << 32) - 1
+        assert (int(ws) > 0) == (built and fits), line
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="libscarfhip.so not built")
+@pytest.mark.parametrize("nq,nr", [(10, 100), (10_000, 10_000)])
+def test_unbuilt_width_is_refused(nq, nr):
+    """Checked before anything is launched, so the pointers are never followed."""
+    L = _lib.lib()
+    p = 4096
+    rc = L.sh_knn_pool(p, nq, p, nr, 128, _lib.SH_BF16, 64, p, p, p, 256, None)
+    assert rc == _lib.SH_EUNSUPPORTED
+    assert b"packed K=144 not supported" in L.sh_last_error()
