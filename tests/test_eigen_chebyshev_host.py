@@ -157,3 +157,20 @@ def test_block_layout():
     assert eigen.chebyshev_block_size(11, 40) == 27
     assert [eigen._block_ld(b) for b in (1, 16, 17, 94, 128, 129, 187, 256)] == \
         [16, 16, 32, 96, 128, 160, 192, 256]
+
+
+@pytest.mark.parametrize("kind,d,n_top", [("pca", 500, 51), ("pca", 700, 21), ("pca", 600, 101),
+                                          ("gram", 800, 21)])
+def test_chebyshev_goes_on_to_rounding(kind, d, n_top):
+    """A solve ends at a few roundings of the largest eigenvalue, not somewhere below its
+    tolerance of 1e-12: 0.003 of that where filtering still helps, and the residual's own
+    rounding (sqrt(d) units of 1.1e-16 in the product, twice) on top, together below 1e-14."""
+    if kind == "pca":
+        n_signal, top = {500: (19, 16.0), 700: (5, 40.0), 600: (30, 8.0)}[d]
+        M = _pca_like(d, n_signal, top, seed=d)
+    else:
+        X = np.random.default_rng(d).standard_normal((5000, d)) * np.geomspace(3, 1, d)
+        M = X.T @ X
+    dev = _NumpyBlock(M, n_top, eigen.chebyshev_block_size(n_top, d))
+    _, _, info = eigen.chebyshev_subspace(dev, n_top, 1e-12)
+    assert info.max_residual <= 1e-14
