@@ -307,6 +307,8 @@ def chebyshev_subspace(dev, n_top: int, tol: float, dyn: float = 16.0,
     for it in range(1, max_iter + 1):
         th, res = dev.rayleigh_ritz() if pending is None else pending
         pending = None
+        if not np.all(np.isfinite(res)):
+            raise EigenNotConverged("residuals are not finite")
         need = n_top - locked
         theta_max = max(theta_max, float(th[0]))
         thr = tol * theta_max

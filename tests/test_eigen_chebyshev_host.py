@@ -174,3 +174,17 @@ def test_chebyshev_goes_on_to_rounding(kind, d, n_top):
     dev = _NumpyBlock(M, n_top, eigen.chebyshev_block_size(n_top, d))
     _, _, info = eigen.chebyshev_subspace(dev, n_top, 1e-12)
     assert info.max_residual <= 1e-14
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_chebyshev_reports_residuals_that_overflow(bad):
+    """A matrix whose residuals overflow is one that the caller takes to LAPACK: the solver's
+    own error, not one of the degree's arithmetic."""
+    class Overflow(_NumpyBlock):
+        def rayleigh_ritz(self, generalized=False):
+            w, res = super().rayleigh_ritz(generalized)
+            return w, np.full_like(res, bad)
+
+    M = _pca_like(300, 5, 10.0, seed=5)
+    with pytest.raises(eigen.EigenNotConverged):
+        eigen.chebyshev_subspace(Overflow(M, 21, eigen.chebyshev_block_size(21, 300)), 21, 1e-12)
