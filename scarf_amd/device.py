@@ -4,8 +4,10 @@ and to name the current HIP stream.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import dataclasses
+import threading
 from typing import Optional
 
 import numpy as np
@@ -39,6 +41,15 @@ class Workspace:
     def __init__(self, device="cuda"):
         self.device = device
         self.buf = None
+        self.lock = threading.Lock()
+
+    @contextlib.contextmanager
+    def hold(self, nbytes: int):
+        """The buffer for one library call whose kernels hand results on in it.  A call gives
+        the interpreter away while it queues them, so another thread with the same stream
+        could queue its own in between; the stream keeps the order only of whole calls."""
+        with self.lock:
+            yield self.get(nbytes)
 
     def get(self, nbytes: int):
         nbytes = max(int(nbytes), 256)
@@ -54,8 +65,8 @@ _workspaces = {}
 def workspace(tag: str = "default") -> Workspace:
     key = (tag, torch.cuda.current_stream().cuda_stream)
     ws = _workspaces.get(key)
-    if ws is None:
-        ws = _workspaces[key] = Workspace()
+    if ws is None:  # two threads that get here end up with the same one
+        ws = _workspaces.setdefault(key, Workspace())
     return ws
 
 

@@ -152,3 +152,36 @@ def test_rerank_of_many_queries_equals_few(cuda, D, pool, extra):
     order = np.lexsort((idx[i], d))[:k]
     assert np.array_equal(whole[0][i].cpu().numpy(), idx[i][order])
     assert np.array_equal(whole[1][i].cpu().numpy(), d[order].astype(np.float32))
+
+
+def test_threads_on_one_stream(cuda):
+    """Four threads search on the default stream, with their own sizes (the workspace grows) and
+    queries: the neighbours of a search alone."""
+    import threading
+
+    import torch
+    from scarf_amd.knn import pack_refs, search
+    say("knn threads on one stream")
+    R = torch.from_numpy(_rows(60_000, 50, 41)).cuda()
+    refs = pack_refs(R, "bf16")
+    Q = [torch.from_numpy(_rows(n, 50, 42 + n)).cuda() for n in (300, 2000, 4500, 9000)]
+    want = [search(q, R, refs, 11) for q in Q]
+    torch.cuda.synchronize()
+    got = [[] for _ in Q]
+    start = threading.Barrier(len(Q))
+
+    def work(i):
+        start.wait()
+        for _ in range(20):
+            got[i].append(search(Q[i], R, refs, 11))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(Q))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i, w in enumerate(want):
+        assert len(got[i]) == 20
+        for g in got[i]:
+            assert torch.equal(g[0], w[0]) and torch.equal(g[1], w[1])
