@@ -149,6 +149,7 @@ __global__ void __launch_bounds__(kPackThreads) k_pack(const float *__restrict__
 // from the top (count the values at or below a prefix); the low kTauSkip bits are left set,
 // which only raises the threshold.  Fewer than `rank` finite minima leave it open.
 constexpr int kTauSkip = 4;
+constexpr int kTauSlots = 64 * 32;  // at most
 // Wave sum with DPP lane moves, the same value in every lane.
 __device__ __forceinline__ int wave_sum_i32(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);   // lane ^ 1
@@ -1009,7 +1010,9 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
     p.len1 = align_up((size_t)cdiv(p.m, p.S1), kSliceAlign);
     p.S1 = (int)cdiv(p.m, p.len1);
     p.per = 16 * p.S1 <= 512 ? 8 : 4 * p.S1 <= 512 ? 2 : 1;
-    while (p.per < 8 && p.S1 * 2 * p.per < 4 * p.rank) p.per = p.per == 1 ? 2 : 8;
+    // more where the rank needs them, as many as k_tau takes (its rank is at most 256)
+    while (p.per < 8 && p.S1 * 2 * p.per < 4 * p.rank)
+      p.per = p.per == 1 ? 2 : 16 * p.S1 <= kTauSlots ? 8 : 4;
     p.slots = p.S1 * 2 * p.per;
     int64_t res3;
     if (p.collect) {
@@ -1157,7 +1160,7 @@ extern "C" int sh_knn_pool(const void *qpack, int64_t nq, const void *rpack, int
       else if (p.slots <= 64 * 8)
         SH_TAU(8);
       else
-        SH_TAU(32);
+        SH_TAU(kTauSlots / 64);
 #undef SH_TAU
       SH_LAUNCH_CHECK("k_tau");
     }

@@ -546,7 +546,7 @@ __global__ void __launch_bounds__(256, (screen_minb<Op, K, CAP>())) k_screen(
 // fewer keys to insert (tau_rank in sh_knn.hip).
 //
 // slot_min[q][slice][2 * per]: a lane half keeps 8 minima (each of two accumulator
-// registers, one v_min3 a pair), folded to `per` = 8, 2 or 1 where many slices give slots
+// registers, one v_min3 a pair), folded to `per` = 8, 4, 2 or 1 where many slices give slots
 // enough.
 __device__ __forceinline__ int64_t sample_row(int64_t i, int shift) {
   // hashed place in the window: cells stored in a repeating order must not alias with it
@@ -690,6 +690,9 @@ __global__ void __launch_bounds__(256, (bound_minb<Op, K>())) k_bound(
     if (per == 8) {
 #pragma unroll
       for (int v = 0; v < 8; ++v) o[v] = vmin[g][v];
+    } else if (per == 4) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o[v] = fminf(vmin[g][2 * v], vmin[g][2 * v + 1]);
     } else {
       const float lo = fminf(fminf(vmin[g][0], vmin[g][1]), fminf(vmin[g][2], vmin[g][3]));
       const float hi = fminf(fminf(vmin[g][4], vmin[g][5]), fminf(vmin[g][6], vmin[g][7]));

@@ -185,3 +185,12 @@ def test_threads_on_one_stream(cuda):
         assert len(got[i]) == 20
         for g in got[i]:
             assert torch.equal(g[0], w[0]) and torch.equal(g[1], w[1])
+
+
+@pytest.mark.parametrize("nq,nr", [(100, 30_000), (500, 25_000), (40, 17_000)])
+def test_pool_of_many_slots(cuda, nq, nr):
+    """A pool of 256 in more slices than eight minima a lane half leave slots for."""
+    import torch
+    say("knn pool of many slots", nq, nr)
+    _compare(torch.from_numpy(_rows(nq, 100, 13)).cuda(),
+             torch.from_numpy(_rows(nr, 100, 14)).cuda(), "fp8", 256)

@@ -1,6 +1,8 @@
 """CPU-only: how sh_knn_pool plans a search.  A width or size that is not built is an error of
 the call, as for sh_knn_screen, whatever the size of the search."""
+import concurrent.futures as cf
 import os
+import shutil
 import subprocess
 import sys
 
@@ -9,6 +11,8 @@ import pytest
 from scarf_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "scarf_amd", "csrc")
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 
 # packed widths that sh_knn_{bf16,fp8,f32}.hip build
 WIDTHS = {"SH_BF16": {16 * i for i in range(1, 9)}, "SH_FP8": {64, 128},
@@ -52,3 +56,45 @@ def test_unbuilt_width_is_refused(nq, nr):
     rc = L.sh_knn_pool(p, nq, p, nr, 128, _lib.SH_BF16, 64, p, p, p, 256, None)
     assert rc == _lib.SH_EUNSUPPORTED
     assert b"packed K=144 not supported" in L.sh_last_error()
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    """(plans, slots that k_tau takes): dicts over a grid of the arguments' whole range."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("ROCm toolchain not available")
+    out = tmp_path_factory.mktemp("plan")
+    srcs = [os.path.join(os.path.dirname(__file__), "knn_plan_driver.hip")] + \
+        [os.path.join(CSRC, f"sh_{n}.hip") for n in ("knn_bf16", "knn_fp8", "knn_f32", "common")]
+    flags = ["--offload-arch=gfx950", "--cuda-host-only", "-O1", "-w", "-std=c++17", "-I",
+             os.path.join(ROOT, "include"), "-I", CSRC]
+
+    def compile_one(src):
+        obj = str(out / (os.path.basename(src) + ".o"))
+        r = subprocess.run([HIPCC, *flags, "-c", src, "-o", obj], capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return obj
+
+    with cf.ThreadPoolExecutor(4) as ex:
+        objs = list(ex.map(compile_one, srcs))
+    exe = str(out / "plan")
+    # no device code is built, so its image stays unresolved; nothing here launches a kernel
+    r = subprocess.run([HIPCC, "--hip-link", "--offload-arch=gfx950", *objs,
+                        "-Wl,--unresolved-symbols=ignore-all", "-o", exe],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.returncode, r.stderr[-2000:])
+    *lines, last = r.stdout.splitlines()
+    names = ("dtype D pool nq nr bounded collect rank S1 per slots m S3 cap len3 bytes").split()
+    return [dict(zip(names, map(int, x.split()))) for x in lines], int(last.split()[1])
+
+
+def test_thresholds_take_every_slot(plans):
+    """k_tau looks at all the minima that k_bound writes, and there are as many as its rank."""
+    rows, tau_slots = plans
+    assert len(rows) > 10_000
+    for p in rows:
+        if p["bounded"]:
+            assert p["slots"] == p["S1"] * 2 * p["per"] <= tau_slots, p
+            assert p["per"] in (1, 2, 4, 8) and p["slots"] >= p["rank"], p
