@@ -925,6 +925,9 @@ struct PoolPlan {
 constexpr int kCUs = 256;
 constexpr size_t kSlotBytes = (size_t)1 << 30;
 constexpr size_t kBufBytes = (size_t)4 << 30;
+// k_collect's positions are bytes in 32 bits, and go on counting where a segment is full: half of
+// so many references (a lane half's) are 2^31 bytes of keys, beside less than 2^28 of segments.
+constexpr int64_t kCollectRefs = (int64_t)1 << 29;
 // Second screen: the first kAgain listed queries in kAgainSlices reference slices (a few
 // failed queries must not wait for one workgroup's walk over all references), the rest
 // kAgainBatch at a time in one slice.
@@ -972,7 +975,7 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
   // k_screen: whole calls take 61.7 us with k_screen and 63.5 with k_collect at 100 queries x
   // 100,000 references (BF16, D = 50), 88 and 81 at 1000 x 100,000, 155 and 135 at
   // 1000 x 500,000, 433 and 353 at 4000 x 500,000.
-  p.collect = p.bounded && (double)nq * (double)nr * c_pair >= 5e-6;
+  p.collect = p.bounded && nr <= kCollectRefs && (double)nq * (double)nr * c_pair >= 5e-6;
   p.cap = screen_cap(pool);
   p.S1 = p.S3 = 1;
   p.len3 = align_up((size_t)nr, kSliceAlign);

@@ -98,3 +98,12 @@ def test_thresholds_take_every_slot(plans):
         if p["bounded"]:
             assert p["slots"] == p["S1"] * 2 * p["per"] <= tau_slots, p
             assert p["per"] in (1, 2, 4, 8) and p["slots"] >= p["rank"], p
+
+
+def test_collected_positions_fit_32_bits(plans):
+    """k_collect counts a lane half's keys in bytes from the wave's first segment, in 32 bits: the
+    64 queries' segments and every second reference of a slice passing."""
+    for p in plans[0]:
+        if p["collect"]:
+            last = 64 * p["S3"] * p["cap"] * 8 + (p["len3"] + 1) // 2 * 8
+            assert last < 1 << 32, p
