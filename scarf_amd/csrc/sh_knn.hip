@@ -232,8 +232,13 @@ __global__ void __launch_bounds__(256) k_tau(const float *__restrict__ slot_min,
 //
 // BITS: the segments hold plain float bits above the index (k_collect), not make_key's word.
 // fail (or NULL): queries whose keys are incomplete -- a segment that overflowed, or fewer
-// than `need` keys -- are listed there instead, to be screened again.
+// than `need` keys -- are listed there instead, to be screened again, and so are those with more
+// keys than kMergeRounds times 64 * E (ties spread evenly over many slices): one wave takes 19 us
+// for each such part, and screening 1000 queries again 0.6 to 1.8 ms.  1000 queries x 300,000,
+// half of both one row: 6.9 ms with no limit, 1.3 with one; ties of 15,000 in 0.77 and, were
+// they screened again, 1.49 ms.
 // list (or NULL): positions list_base.. of a list of queries whose length the device knows.
+constexpr int kMergeRounds = 96;
 template <int PE, int E, bool BITS>
 __global__ void __launch_bounds__(256) k_pool_merge(
     const uint64_t *__restrict__ buf, const int32_t *__restrict__ seg_cnt, int64_t n, int S,
@@ -271,7 +276,7 @@ __global__ void __launch_bounds__(256) k_pool_merge(
     const int sg = lane * run + i;
     if (sg < ns) off[sg] += inc - mine;
   }
-  if (fail && (wave_any(over) || total < need)) {
+  if (fail && (wave_any(over) || total < need || total > kMergeRounds * 64 * E)) {
     if (lane == 0) fail[atomicAdd(fail_n, 1)] = fail_base + (int32_t)p;
     return;
   }
@@ -925,8 +930,9 @@ struct PoolPlan {
 constexpr int kCUs = 256;
 constexpr size_t kSlotBytes = (size_t)1 << 30;
 constexpr size_t kBufBytes = (size_t)4 << 30;
-// k_collect's positions are bytes in 32 bits, and go on counting where a segment is full: half of
-// so many references (a lane half's) are 2^31 bytes of keys, beside less than 2^28 of segments.
+// k_collect's positions are bytes in 32 bits.  A lane half stops where its segment is full, but
+// for keys of minus infinity, which pass any threshold: half of so many references (a lane
+// half's) are 2^31 bytes of keys, beside less than 2^28 of segments.
 constexpr int64_t kCollectRefs = (int64_t)1 << 29;
 // Second screen: the first kAgain listed queries in kAgainSlices reference slices (a few
 // failed queries must not wait for one workgroup's walk over all references), the rest

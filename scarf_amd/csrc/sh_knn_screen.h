@@ -19,7 +19,9 @@
 // 32 x 32 tile is filtered with a 16-value min tree and one compare per query;
 // only tiles with a hit (rare once tau has settled) take the insertion path.  When
 // a buffer nears CAP the owning wave sorts it (bitonic across the wave) and keeps
-// the best `pool`.  Each wave owns its queries, so no cross-wave synchronisation.
+// the best `pool`.  References come in index order and the lower index wins a tie, so from
+// then on tau excludes the pool-th key itself: a query with many equal references would
+// otherwise insert them all.  Each wave owns its queries, so no cross-wave synchronisation.
 // Optionally each query block first screens a set of seed reference rows (for self
 // queries in locality order: the block's own rows) and starts tau at their pool-th key.
 #pragma once
@@ -496,7 +498,8 @@ __global__ void __launch_bounds__(256, (screen_minb<Op, K, CAP>())) k_screen(
                                                nullptr, nullptr, tnew);
             if (n == src) {
               cnt[g] = h == 0 ? (keep + 1) / 2 : keep - (keep + 1) / 2;
-              tau[g] = fminf(tau[g], tnew);
+              // what comes now has a higher index, so of equal keys none can enter any more
+              if (tnew < kOpen) tau[g] = fminf(tau[g], ord_float(float_ord(tnew) - 1));
             }
           }
         }
@@ -714,7 +717,9 @@ __global__ void __launch_bounds__(256, (bound_minb<Op, K>())) k_bound(
 // segment (cap / 2 words of reference index and key bits) and is counted.  k_pool_merge selects
 // the pool; a query whose segment overflowed, or that met fewer than `pool` keys (its
 // threshold was a guess from a sample), goes on a list and is screened again from an open
-// threshold.  Without the compaction the loop is a tenth of k_screen's code and keeps its
+// threshold.  A lane half whose segment overflowed collects nothing more: 100,000 cells of
+// which half are one row take 6.1 ms in all, with that and k_screen's rule for equal keys (155
+// without both, 84 in one scan by a k_screen that inserts them all).  Without the compaction the loop is a tenth of k_screen's code and keeps its
 // registers (122 of 128, no spills, against 43 spilled).  262,144 queries x 1,048,576
 // references of 64 BF16 elements: 28.0 ms with no key passing (1.26 PFLOP/s; k_screen 31.1),
 // 32.3 ms with 213 keys per query.  The loop without filter, LDS reads and staging takes
@@ -890,6 +895,8 @@ __global__ void __launch_bounds__(256, (collect_minb<Op, K>())) k_collect(
               }
             }
           }
+          // past the room the query is screened again, whatever else it meets
+          if ((int)(pos[g] - last[g]) > 8) tau[g] = -INFINITY;
         }
       }
     }

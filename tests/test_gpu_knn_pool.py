@@ -194,3 +194,65 @@ def test_pool_of_many_slots(cuda, nq, nr):
     say("knn pool of many slots", nq, nr)
     _compare(torch.from_numpy(_rows(nq, 100, 13)).cuda(),
              torch.from_numpy(_rows(nr, 100, 14)).cuda(), "fp8", 256)
+
+
+@pytest.mark.parametrize("screen,pool,D,nq,nr,equal", [
+    ("bf16", 64, 50, 1, 3000, 200), ("bf16", 64, 50, 300, 20_000, 10_000),
+    ("bf16", 64, 50, 700, 300_000, 150_000), ("bf16", 128, 50, 9000, 60_000, 5000),
+    ("fp32", 64, 50, 500, 30_000, 15_000), ("fp8", 256, 100, 300, 40_000, 9000)])
+def test_equal_references_keep_the_lowest_indices(cuda, screen, pool, D, nq, nr, equal):
+    """Queries that are one of many equal references: its pool is the lowest-indexed of them,
+    whichever of the scan's ways it takes (the second screen, ties in every slice, one slice)."""
+    import torch
+    from scarf_amd import _lib
+    from scarf_amd.device import ptr, stream_handle
+    from scarf_amd.knn import pack, pack_refs
+    say("knn equal references", screen, pool, nq, nr, equal)
+    L, code = _lib.lib(), _lib.DTYPES[screen]
+    R = _rows(nr, D, 31)
+    at = np.sort(np.random.default_rng(32).choice(nr, equal, replace=False))
+    R[at] = 3.0 * R[at[0]]  # far out, so that nothing else is near
+    R = torch.from_numpy(R).cuda()
+    Q = torch.from_numpy(_rows(nq, D, 33)).cuda()
+    Q[::2] = R[int(at[0])]
+    refs = pack_refs(R, screen)
+    qp, _, _ = pack(Q, screen, 1)
+    want = torch.from_numpy(at[:pool].astype(np.int64)).cuda()
+    for name in ("sh_knn_pool", "sh_knn_screen"):
+        cand = torch.full((nq, pool), -1, dtype=torch.int64, device="cuda")
+        cnt = torch.empty(nq, dtype=torch.int32, device="cuda")
+        need = (L.sh_knn_pool_workspace(nq, nr, D, code, pool) if name == "sh_knn_pool" else
+                L.sh_knn_screen_workspace(nq, pool, 1))
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        extra = () if name == "sh_knn_pool" else (1, None)
+        aux = () if name == "sh_knn_pool" else (None, None)
+        _lib.call(name, ptr(qp), nq, ptr(refs.data), nr, D, code, *aux, pool, *extra, ptr(cand),
+                  ptr(cnt), ptr(ws), need, stream_handle())
+        assert bool((cnt == pool).all())
+        assert bool(((cand[::2] & 0xffffffff) == want[None, :]).all())
+
+
+def test_equal_references_are_not_a_slow_case(cuda):
+    """100,000 cells of which half are one row, against the same number without equal ones:
+    about 2.2 times the time where every tie was inserted, twice, it was 57 times."""
+    import time
+
+    import torch
+    from scarf_amd.knn import pack_refs, search
+    say("knn time with equal references")
+    E = torch.from_numpy(_rows(100_000, 50, 34)).cuda()
+    T = E.clone()
+    T[torch.randperm(100_000, device="cuda")[:50_000]] = E[0]
+    took = []
+    for x in (E, T):
+        refs = pack_refs(x, "bf16")
+        best = float("inf")
+        for _ in range(4):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            search(x, x, refs, 11, self_offset=0)
+            torch.cuda.synchronize()
+            best = min(best, time.perf_counter() - t)
+        took.append(best)
+    say("ms", [1e3 * t for t in took])
+    assert took[1] < 10.0 * took[0]
