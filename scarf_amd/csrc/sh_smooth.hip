@@ -110,15 +110,21 @@ __device__ __forceinline__ float smooth_rho(const float (&d)[KM], float lc) {
 // steps (hardware exp and reciprocal) place the root to about 1e-7; within 5e-5 / slope of
 // it, five times the stop tolerance, a step evaluates the sum as before, so every midpoint,
 // and the sigma, is the one that the plain bisection gives.  Where Newton does not settle
-// (no root, a flat sum, non-finite distances) every step evaluates.  gap[j] = d[j] - rho,
+// (a flat sum, non-finite distances) every step evaluates.  gap[j] = d[j] - rho,
 // infinite past the row's k distances: no test of j < k (their masks did not fit the scalar
 // registers), and a term of exactly zero.
 template <int KM>
 __device__ __forceinline__ float smooth_sigma(const float (&gap)[KM], int32_t k, double target,
                                               int32_t n_iter) {
   float root = 0.f, near = INFINITY;
-  {
-    const float t = (float)target;
+  // Rows without a root decide the same way at every step: 64 evaluations of each, with the
+  // padded terms, took 1M rows of 2 from 0.21 to 0.51 ms.  0.01 is far more than the sums'
+  // rounding and the tolerance.
+  const float t = (float)target;
+  if ((float)(k - 1) < t - 0.01f) {  // the sum is below the target
+    root = INFINITY;
+    near = 0.f;
+  } else {
     float gaps = 0.f;
 #pragma unroll
     for (int j = 1; j < KM; ++j) gaps += gap[j] < INFINITY ? fmaxf(gap[j], 0.f) : 0.f;
@@ -142,6 +148,21 @@ __device__ __forceinline__ float smooth_sigma(const float (&gap)[KM], int32_t k,
         break;
       }
       x *= __builtin_amdgcn_exp2f(step * 1.44269504f);
+    }
+    if (near == INFINITY) {
+      int ones = 0, less = 0;  // terms of 1 whatever sigma, and of less than that
+#pragma unroll
+      for (int j = 1; j < KM; ++j) {
+        ones += !(gap[j] > 0.f);
+        less += gap[j] > 0.f && gap[j] < INFINITY;
+      }
+      if ((float)ones > t + 0.01f) {
+        root = -1.f;
+        near = 0.f;
+      } else if ((float)(ones + less) < t - 0.01f) {
+        root = INFINITY;
+        near = 0.f;
+      }
     }
   }
   float lo = 0.f, hi = INFINITY, mid = 1.f;
