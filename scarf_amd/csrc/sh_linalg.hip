@@ -854,8 +854,17 @@ extern "C" int sh_dgemm(int transA, int64_t m, int64_t n, int64_t k, double alph
          "sh_dgemm: leading dimension too small");
   SH_ARG(cdiv(n, kDT) <= 0x7fffffff && cdiv(m, kDT) <= 65535, "sh_dgemm: matrix too large");
   if (m == 0 || n == 0) return SH_OK;
-  // narrow products of many rows; below that (or wider) the 64 x 64 tiles fill the GPU
-  if (!transA && n <= kTallMax && k <= kTallMax && m >= 256 && cdiv(m, 16) <= 0x7fffffff) {
+  // Where the 64 x 64 tiles leave CUs idle, or hold padding (3 of 8 columns; a quarter, up to
+  // the rows where their reuse of A wins all the same), or have next to nothing to reuse.  us with tiles / without:
+  // n = k = 64 9.4 / 5.0 at 2000 rows, 10.1 / 7.5 at 8000, 10.9 / 12.5 at 16,000 and 150 / 172 at
+  // 300,000; 94 13.3 / 5.7, 22 / 18 at 16,000, 136 / 114 at 128,000, 351 / 387 at 300,000;
+  // 128 17.1 / 11.7 at 3000, 17.9 / 21 at 8000; 256 31 / 21 at 2000, 53 / 72 at 8000 and
+  // 324 / 557 at 64,000; n = 200, k = 8 176 / 146 and n = 8, k = 200 357 / 124 at 300,000.
+  const int64_t tiles = cdiv(m, kDT) * cdiv(n, kDT);
+  const size_t used = align_up(n, 16), held = align_up(n, kDT);
+  const bool padded = 8 * used <= 5 * held || (4 * used <= 3 * held && m <= 1 << 17);
+  if (!transA && n <= kTallMax && k <= kTallMax && m >= 256 && cdiv(m, 16) <= 0x7fffffff &&
+      (tiles <= 200 || padded || k <= 16)) {
     hipLaunchKernelGGL(k_dgemm_tall, dim3((uint32_t)cdiv(m, 16), (uint32_t)cdiv(n, 64)),
                        dim3(256), 0, (hipStream_t)stream, m, (int32_t)n, (int32_t)k, A, lda, B,
                        ldb, alpha, beta, C, ldc);

@@ -78,3 +78,10 @@ def test_merge_matrix_edges(cuda, d, nc, first):
         mag = mag + (np.abs(V).T * s2) @ np.abs(V) + np.outer(np.abs(mc), np.abs(mc))
     assert np.all(np.abs(got - want) <= (nc + 6) * 2.0 ** -52 * mag)
     assert np.array_equal(got, got.T)
+
+
+@pytest.mark.parametrize("m,n,k", [(12_800, 64, 64), (12_801, 64, 64), (20_000, 94, 94),
+                                   (20_000, 200, 16), (20_000, 200, 17)])
+def test_gemm_of_many_rows(cuda, m, n, k):
+    """Both kernels' sides of the lines in tiles, padding and depth."""
+    test_tall_gemm(cuda, m, n, k)
