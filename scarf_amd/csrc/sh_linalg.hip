@@ -153,6 +153,25 @@ __global__ void __launch_bounds__(256) k_dgemm_tall(int64_t m, int32_t n, int32_
 // kMmC rows at a time: one thread per entry re-read both strips for every entry (166 us at
 // d = 2000, 51 components; now 43).
 constexpr int kMmT = 64, kMmC = 32;
+// One thread per entry, for small matrices and none or few components: us with tiles / entries,
+// 51 components 16 / 8 at d = 200, 16 / 11 at 400 and 16 / 21 at 600; 11 components 8.7 / 7.1
+// at 600, 9.1 / 10.7 at 800; none 5.3 / 4.0 at 800 and 234 / 220 at 8000.
+__global__ void __launch_bounds__(256) k_merge_entries(
+    const double *__restrict__ G, int32_t d, double n, const double *__restrict__ bm,
+    const double *__restrict__ Vt, const double *__restrict__ s2, int32_t nc,
+    const double *__restrict__ mc, double *__restrict__ M) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= (int64_t)d * d) return;
+  const int i = (int)(e / d), j = (int)(e % d);
+  double x = G[e] - n * (bm[i] * bm[j]);
+  if (Vt) {
+    double r = 0.0;
+    for (int c = 0; c < nc; ++c) r += s2[c] * (Vt[(int64_t)c * d + i] * Vt[(int64_t)c * d + j]);
+    x += r;
+  }
+  if (mc) x += mc[i] * mc[j];
+  M[e] = x;
+}
 __global__ void __launch_bounds__(256) k_merge_matrix(
     const double *__restrict__ G, int32_t d, double n, const double *__restrict__ bm,
     const double *__restrict__ Vt, const double *__restrict__ s2, int32_t nc,
@@ -161,31 +180,29 @@ __global__ void __launch_bounds__(256) k_merge_matrix(
   const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
   const int i0 = blockIdx.y * kMmT, j0 = blockIdx.x * kMmT;
   double r[4][4] = {};
-  if (Vt) {
-    for (int c0 = 0; c0 < nc; c0 += kMmC) {
-      const int cn = min(kMmC, nc - c0);
-      for (int e = tid; e < cn * kMmT; e += 256) {
-        const int c = e / kMmT, t = e % kMmT;
-        const double *row = Vt + (int64_t)(c0 + c) * d;
-        vi[c][t] = i0 + t < d ? row[i0 + t] : 0.0;
-        vj[c][t] = j0 + t < d ? row[j0 + t] : 0.0;
-      }
-      __syncthreads();
-      for (int c = 0; c < cn; ++c) {
-        const double sc = s2[c0 + c];
-        double a[4], b[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          a[u] = vi[c][ty + 16 * u];
-          b[u] = vj[c][tx + 16 * u];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) r[u][v] += sc * (a[u] * b[v]);
-      }
-      __syncthreads();
+  for (int c0 = 0; c0 < nc; c0 += kMmC) {
+    const int cn = min(kMmC, nc - c0);
+    for (int e = tid; e < cn * kMmT; e += 256) {
+      const int c = e / kMmT, t = e % kMmT;
+      const double *row = Vt + (int64_t)(c0 + c) * d;
+      vi[c][t] = i0 + t < d ? row[i0 + t] : 0.0;
+      vj[c][t] = j0 + t < d ? row[j0 + t] : 0.0;
     }
+    __syncthreads();
+    for (int c = 0; c < cn; ++c) {
+      const double sc = s2[c0 + c];
+      double a[4], b[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a[u] = vi[c][ty + 16 * u];
+        b[u] = vj[c][tx + 16 * u];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) r[u][v] += sc * (a[u] * b[v]);
+    }
+    __syncthreads();
   }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
@@ -196,7 +213,7 @@ __global__ void __launch_bounds__(256) k_merge_matrix(
       if (i < d && j < d) {
         const int64_t e = (int64_t)i * d + j;
         double x = G[e] - n * (bm[i] * bm[j]);
-        if (Vt) x += r[u][v];
+        x += r[u][v];
         if (mc) x += mc[i] * mc[j];
         M[e] = x;
       }
@@ -884,8 +901,13 @@ extern "C" int sh_merge_matrix(const double *G, int32_t d, double n, const doubl
   SH_ARG(d > 0 && G && bm && M, "sh_merge_matrix: bad arguments");
   SH_ARG(!Vt || (s2 && nc > 0), "sh_merge_matrix: Vt needs s2 and nc > 0");
   const uint32_t t = (uint32_t)cdiv(d, kMmT);
-  hipLaunchKernelGGL(k_merge_matrix, dim3(t, t), dim3(256), 0, (hipStream_t)stream, G, d, n, bm,
-                     Vt, s2, nc, mc, M);
+  const int64_t n2 = (int64_t)d * d;
+  if (!Vt || d <= 400 || n2 * nc <= 4000000)
+    hipLaunchKernelGGL(k_merge_entries, dim3((uint32_t)cdiv(n2, 256)), dim3(256), 0,
+                       (hipStream_t)stream, G, d, n, bm, Vt, s2, nc, mc, M);
+  else
+    hipLaunchKernelGGL(k_merge_matrix, dim3(t, t), dim3(256), 0, (hipStream_t)stream, G, d, n, bm,
+                       Vt, s2, nc, mc, M);
   SH_LAUNCH_CHECK("k_merge_matrix");
   return SH_OK;
 }

@@ -80,6 +80,12 @@ def test_merge_matrix_edges(cuda, d, nc, first):
     assert np.array_equal(got, got.T)
 
 
+@pytest.mark.parametrize("d,nc", [(401, 51), (640, 9), (640, 10), (1200, 3)])
+def test_merge_matrix_tiles(cuda, d, nc):
+    """Past 400 features and a few million products the tiled kernel, on both sides of the line."""
+    test_merge_matrix_edges(cuda, d, nc, False)
+
+
 @pytest.mark.parametrize("m,n,k", [(12_800, 64, 64), (12_801, 64, 64), (20_000, 94, 94),
                                    (20_000, 200, 16), (20_000, 200, 17)])
 def test_gemm_of_many_rows(cuda, m, n, k):
