@@ -351,8 +351,13 @@ __device__ __forceinline__ float project_delta(uint32_t v, int32_t c, bool there
   }
   return xv * is;
 }
-// steps (of four entries) whose loads are all in flight before the first is used
+// steps (of four entries) whose loads are all in flight before the first is used; with two loads a
+// step half of that, since the registers of eight leave a SIMD four waves instead of six, but
+// where a launch is at most two fills of those (us with eight / four steps at D = 128: 1000 x 2000
+// at 8% 16.7 / 19, 100,000 at 2% 147 / 126, 300,000 at 0.5% 299 / 231, at 8% 1229 / 1230; with
+// library sizes in the kernel 23.7 / 26.9, 167 / 136, 358 / 268, 1409 / 1198)
 constexpr int kProjSteps = 8;
+constexpr int64_t kProjFewRows = 256 * 32;
 // W's address for a lane: `at` is the entry's byte offset (its row index if WIDE), `lo` the
 // lane's own
 template <bool WIDE>
@@ -380,8 +385,8 @@ __device__ __forceinline__ void project_steps(std::integer_sequence<int, I...>, 
                                               const uint32_t (&lo)[DPL], const char *W,
                                               int64_t row_bytes, float4 (&acc)[DPL]) {
   constexpr uint64_t kStep = 0x0001000100010001ull;  // lane 0 of each group
-  constexpr uint64_t kAll = (((1ull << kProjSteps) - 1) << B) * kStep;
-  float4 w[kProjSteps][DPL];
+  constexpr uint64_t kAll = (((1ull << sizeof...(I)) - 1) << B) * kStep;
+  float4 w[sizeof...(I)][DPL];
   if ((valid & kAll) == kAll) {
     (
         [&] {
@@ -433,7 +438,7 @@ __device__ __forceinline__ void project_store(float4 (&acc)[DPL], const bool (&c
     }
   }
 }
-template <int DPL, bool WIDE>
+template <int DPL, bool WIDE, int STEPS>
 __global__ void __launch_bounds__(256) k_project(
     const uint32_t *__restrict__ vals, const int32_t *__restrict__ cols,
     const int64_t *__restrict__ rowptr, int64_t n_rows, const int32_t *__restrict__ col_map,
@@ -483,10 +488,16 @@ __global__ void __launch_bounds__(256) k_project(
                                       inv_sigma, 1, clip, &f);
     const uint64_t valid = __ballot(f >= 0);
     const int at = WIDE ? f : (int)((uint32_t)f * (uint32_t)row_bytes);
-    const auto seq = std::make_integer_sequence<int, kProjSteps>{};
+    const auto seq = std::make_integer_sequence<int, STEPS>{};
     project_steps<DPL, WIDE, 0>(seq, at, delta, valid, lo, Wb, row_bytes, acc);
-    if (b - t0 > 4 * kProjSteps)
-      project_steps<DPL, WIDE, kProjSteps>(seq, at, delta, valid, lo, Wb, row_bytes, acc);
+    if (b - t0 > 4 * STEPS)
+      project_steps<DPL, WIDE, STEPS>(seq, at, delta, valid, lo, Wb, row_bytes, acc);
+    if constexpr (STEPS == 4) {
+      if (b - t0 > 8 * STEPS)
+        project_steps<DPL, WIDE, 2 * STEPS>(seq, at, delta, valid, lo, Wb, row_bytes, acc);
+      if (b - t0 > 12 * STEPS)
+        project_steps<DPL, WIDE, 3 * STEPS>(seq, at, delta, valid, lo, Wb, row_bytes, acc);
+    }
     c = cn;
     v = vn;
   }
@@ -905,8 +916,11 @@ extern "C" int sh_project(const uint32_t *vals, const int32_t *cols, const int64
     SH_LAUNCH_CHECK("k_project_hot");
     return SH_OK;
   }
-  auto kern = D <= 64 ? (wide ? k_project<1, true> : k_project<1, false>)
-                      : (wide ? k_project<2, true> : k_project<2, false>);
+  constexpr int kS = kProjSteps;
+  auto kern = D <= 64                  ? (wide ? k_project<1, true, kS> : k_project<1, false, kS>)
+              : n_rows <= kProjFewRows ? (wide ? k_project<2, true, kS> : k_project<2, false, kS>)
+                                       : (wide ? k_project<2, true, kS / 2>
+                                               : k_project<2, false, kS / 2>);
   hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, vals, cols, rowptr, n_rows,
                      col_map, n_cols_in, (float)sf, log_transform, libsize, mu, inv_sigma, clip, W,
                      ldw, D, c, E_out, lde);

@@ -145,3 +145,29 @@ def test_stats_values_over_the_range(cuda, sf):
     # the quotient within half a unit in the last place, of which a logarithm passes on at most
     # as much, and the logarithm within one, on both sides: 3 units, each at most 2^-52
     np.testing.assert_allclose(st.chunk_sums.cpu().numpy(), x, rtol=3 * 2.0 ** -52, atol=0)
+
+
+@pytest.mark.parametrize("D", [65, 128])
+@pytest.mark.parametrize("mapped", [False, True])
+def test_project_of_many_rows_equals_few(cuda, D, mapped):
+    """Past 8192 rows the second pass of columns takes fewer steps at once: the same bits as for
+    pieces of fewer rows, over rows that end in each of a batch's four blocks."""
+    import torch
+
+    from scarf_amd.device import DeviceCSR, col_map_tensor
+    from scarf_amd.normalize import NormParams
+    from scarf_amd.pca import Projector
+    say("project rows", D, mapped)
+    d_in, n = 400, 8197
+    csr = DeviceCSR.from_host(_csr(n, d_in, (0, 1, 15, 16, 17, 31, 33, 47, 49, 63, 64, 65, 130), 9))
+    rng = np.random.default_rng(10)
+    keep = np.sort(rng.choice(d_in, 250, replace=False)) if mapped else np.arange(d_in)
+    d = keep.shape[0]
+    cm, _ = col_map_tensor(d_in, keep if mapped else None)
+    proj = Projector.build(rng.standard_normal((d, D)), rng.uniform(0.1, 1.0, d),
+                           rng.uniform(0.5, 2.0, d), clip=3.0)
+    E = proj.project(csr, NormParams(), col_map=cm)
+    for a in range(0, n, 4000):
+        m = min(4000, n - a)
+        part = proj.project(csr, NormParams(), col_map=cm, row_start=a, n_rows=m)
+        assert torch.equal(E[a:a + m].view(torch.int32), part.view(torch.int32))
