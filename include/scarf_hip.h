@@ -218,6 +218,14 @@ int sh_project(const uint32_t *vals, const int32_t *cols, const int64_t *rowptr,
                double sf, int log_transform, const double *libsize, const float *mu,
                const float *inv_sigma, float clip, const float *W, int64_t ldw,
                int32_t D, const float *c, float *E_out, int64_t lde, sh_stream_t stream);
+/* The same for a caller that knows how many entries the rows hold, all in all or about (negative:
+ * not known); that only chooses between kernels of the same results. */
+int sh_project_counted(const uint32_t *vals, const int32_t *cols, const int64_t *rowptr,
+                       int64_t n_rows, int64_t n_entries, const int32_t *col_map,
+                       int32_t n_cols_in, int32_t d, double sf, int log_transform,
+                       const double *libsize, const float *mu, const float *inv_sigma,
+                       float clip, const float *W, int64_t ldw, int32_t D, const float *c,
+                       float *E_out, int64_t lde, sh_stream_t stream);
 
 /* ---- k nearest neighbours (squared L2) ------------------------------------------
  * Replaces hnswlib.Index (ann.py:14-28, 194-205, 290-326) with an exact screen:

@@ -59,6 +59,8 @@ _SIGS = {
     "sh_dense_z": (_int, [_p, _int, _i64, _i32, _i64, _p, _p, _f64, _p, _i64, _p]),
     "sh_dense_project": (_int, [_p, _int, _i64, _i32, _i64, _p, _p, _f64, _p, _i32, _p, _i64, _p]),
     "sh_project": (_int, [_p, _p, _p, _i64, _p, _i32, _i32, _f64, _int, _p, _p, _p, _f32, _p, _i64, _i32, _p, _p, _i64, _p]),
+    "sh_project_counted": (_int, [_p, _p, _p, _i64, _i64, _p, _i32, _i32, _f64, _int, _p, _p, _p, _f32, _p, _i64,
+                                  _i32, _p, _p, _i64, _p]),
     "sh_knn_pack_k": (_i32, [_int, _i32]),
     "sh_knn_pack_row_bytes": (_i64, [_int, _i32]),
     "sh_knn_pack": (_int, [_p, _i64, _i32, _i64, _int, _int, _p, _p, _p]),

@@ -527,12 +527,21 @@ constexpr int kHotThreads = 1024;
 constexpr int kHotBlocks = 256;  // one a CU
 constexpr int kHotSample = 4;    // rows a wave samples for the counts
 // Building the table costs 15-70 us a launch, more with more features, so it takes 32 rows a
-// wave to pay: at 131,072 rows 111 us against 108 at 600 features and 8%, 145 / 157 at 1000,
+// wave to pay: at 8% non-zeros and 131,072 rows 111 us against 108 at 600 features and 8%, 145 / 157 at 1000,
 // 239 / 279 at 2000, 511 / 700 at 4000 (8%) and 527 / 699 at 6000, 746 / 923 at 8000 (5%); at
 // half as many rows 64 / 58, 139 / 148, 261 / 291.  Beyond 8192 features the means and places
 // leave less than half of LDS to the table.
 constexpr int64_t kHotRows = (int64_t)kHotBlocks * (kHotThreads / 64) * 32;
 constexpr int kHotMaxD = 8192;
+// A row costs more too (1.1 ns against 0.45 in k_project, where 32 waves a CU share the row's own
+// loads instead of 16; 0.7 against 0.35 if the library sizes are given) and an entry less, so rows
+// have to be long enough, where the caller says how long they are.  us with the table / without,
+// 2000 features, library sizes given: 500,000 rows of 10 entries 292 / 241, of 40 420 / 415, of 80
+// 610 / 769; 131,072 rows of 40 117 / 103, of 80 162 / 167, of 160 255 / 295.  Summed in the
+// kernel: 500,000 rows of 40 563 / 472, of 80 847 / 910; 131,072 of 80 218 / 195, of 160 342 / 341.
+constexpr bool hot_entries(int64_t n_rows, int64_t entries, bool libsize) {
+  return entries >= (libsize ? 28 * n_rows + 4000000 : 60 * n_rows + 8000000);
+}
 
 // explicitly LDS: through a generic pointer the compiler joins the two sources of an entry's
 // row into one flat load
@@ -897,6 +906,18 @@ extern "C" int sh_project(const uint32_t *vals, const int32_t *cols, const int64
                           const float *inv_sigma, float clip, const float *W, int64_t ldw,
                           int32_t D, const float *c, float *E_out, int64_t lde,
                           sh_stream_t stream) {
+  return sh_project_counted(vals, cols, rowptr, n_rows, -1, col_map, n_cols_in, d, sf,
+                            log_transform, libsize, mu, inv_sigma, clip, W, ldw, D, c, E_out, lde,
+                            stream);
+}
+
+extern "C" int sh_project_counted(const uint32_t *vals, const int32_t *cols,
+                                  const int64_t *rowptr, int64_t n_rows, int64_t n_entries,
+                                  const int32_t *col_map, int32_t n_cols_in, int32_t d, double sf,
+                                  int log_transform, const double *libsize, const float *mu,
+                                  const float *inv_sigma, float clip, const float *W, int64_t ldw,
+                                  int32_t D, const float *c, float *E_out, int64_t lde,
+                                  sh_stream_t stream) {
   SH_ARG(n_rows >= 0 && d > 0 && D > 0 && D <= 128 && ldw >= D && lde >= D,
          "sh_project: bad sizes d=%d D=%d ldw=%lld lde=%lld", d, D, (long long)ldw,
          (long long)lde);
@@ -908,7 +929,8 @@ extern "C" int sh_project(const uint32_t *vals, const int32_t *cols, const int64
   dim3 grid(cdiv(n_rows, 4)), block(256);
   // byte offsets into W in 32 bits, if it is that small
   const bool wide = (uint64_t)d * (uint64_t)ldw * 4 > 0xffffffffull;
-  if (D <= 64 && n_rows >= kHotRows && d <= kHotMaxD && !wide) {
+  if (D <= 64 && n_rows >= kHotRows && d <= kHotMaxD && !wide &&
+      (n_entries < 0 || hot_entries(n_rows, n_entries, libsize != nullptr))) {
     hipLaunchKernelGGL(col_map ? k_project_hot<true> : k_project_hot<false>, dim3(kHotBlocks),
                        dim3(kHotThreads), 0, (hipStream_t)stream, vals, cols, rowptr, n_rows,
                        col_map, n_cols_in, d, (float)sf, log_transform, libsize, mu, inv_sigma,

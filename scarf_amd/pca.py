@@ -422,8 +422,9 @@ class Projector:
             out = torch.empty((n_rows, self.D), dtype=torch.float32, device=csr.rowptr.device)
         if n_rows == 0:
             return out
-        _lib.call("sh_project", ptr(csr.vals), ptr(csr.cols), ptr(csr.rowptr, row_start), n_rows,
-                  ptr(col_map), csr.n_cols, self.d, float(params.size_factor),
+        entries = csr.nnz * n_rows // max(csr.n_rows, 1)  # about, for a part of the rows
+        _lib.call("sh_project_counted", ptr(csr.vals), ptr(csr.cols), ptr(csr.rowptr, row_start),
+                  n_rows, entries, ptr(col_map), csr.n_cols, self.d, float(params.size_factor),
                   int(params.log_transform),
                   ptr(libsize, row_start) if libsize is not None else None, ptr(self.mu),
                   ptr(self.inv_sigma), self.clip, ptr(self.W), self.W.stride(0), self.D,

@@ -171,3 +171,48 @@ def test_project_of_many_rows_equals_few(cuda, D, mapped):
         m = min(4000, n - a)
         part = proj.project(csr, NormParams(), col_map=cm, row_start=a, n_rows=m)
         assert torch.equal(E[a:a + m].view(torch.int32), part.view(torch.int32))
+
+
+@pytest.mark.parametrize("d_in,D,clip,mapped,sizes", [
+    (3, 1, 0.0, False, True), (40, 64, 3.0, False, False), (2500, 50, 3.0, True, False),
+    (2500, 33, 0.0, False, True), (8192, 64, 3.0, False, True)])
+def test_project_table_and_entries(cuda, d_in, D, clip, mapped, sizes):
+    """sh_project takes the table of W's rows from 131,072 rows on; the caller's count of entries
+    can say that rows are too short for it.  The same bits, with all of W in the table and with
+    part of it, empty and long rows, counts on both sides of 64 and an infinity in W."""
+    import torch
+
+    from scarf_amd import _lib
+    from scarf_amd.device import DeviceCSR, col_map_tensor, ptr, stream_handle
+    from scarf_amd.pca import Projector
+    from scarf_amd.synth import CSR
+    say("project table", d_in, D, clip, mapped, sizes)
+    rng = np.random.default_rng(18)
+    n = 131072 + 5
+    ln = np.minimum(np.array([0, 1, 31, 33, 64, 65, 5, 2, 9, 20])[np.arange(n) % 10], d_in)
+    ln[[7, 70_000, n - 1]] = min(d_in, 1000)
+    rp = np.concatenate([[0], np.cumsum(ln)]).astype(np.int64)
+    within = np.arange(rp[-1]) - np.repeat(rp[:-1], ln)
+    gap = np.maximum(d_in // np.maximum(np.repeat(ln, ln), 1), 1)
+    cols = np.minimum(within * gap + (rng.random(rp[-1]) ** 3 * gap).astype(np.int64), d_in - 1)
+    vals = np.where(rng.random(rp[-1]) < 0.02, rng.integers(60, 5000, rp[-1]),
+                    rng.integers(1, 8, rp[-1])).astype(np.uint32)
+    csr = DeviceCSR.from_host(CSR(vals, cols.astype(np.int32), rp, d_in))
+    keep = np.sort(rng.choice(d_in, d_in // 2, replace=False)) if mapped else np.arange(d_in)
+    d = keep.shape[0]
+    W = rng.standard_normal((d, D))
+    W[d // 2, 0] = np.inf
+    cm, _ = col_map_tensor(d_in, keep if mapped else None)
+    p = Projector.build(W, rng.uniform(0.1, 1.0, d), rng.uniform(0.5, 2.0, d), clip=clip)
+    p.c.zero_()  # finite: the infinity of W stays in the rows that use it
+    lib = torch.rand(n, dtype=torch.float64, device="cuda") * 900 + 100 if sizes else None
+    out = []
+    for name, count in (("sh_project", ()), ("sh_project_counted", (0,)),
+                        ("sh_project_counted", (1 << 40,)), ("sh_project_counted", (-1,))):
+        E = torch.full((n, D), -7.0, device="cuda")
+        _lib.call(name, ptr(csr.vals), ptr(csr.cols), ptr(csr.rowptr), n, *count, ptr(cm), d_in, d,
+                  1000.0, 1, ptr(lib), ptr(p.mu), ptr(p.inv_sigma), p.clip, ptr(p.W),
+                  p.W.stride(0), D, ptr(p.c), ptr(E), D, stream_handle())
+        out.append(E.view(torch.int32))
+    for E in out[1:]:
+        assert torch.equal(out[0], E)
