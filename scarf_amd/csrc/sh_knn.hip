@@ -971,7 +971,12 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
   PoolPlan p = {};
   const KnnOps ops = knn_ops(dtype);
   const int64_t qb = std::max<int64_t>(1, cdiv(nq, 256));
-  p.bounded = nr >= 8 * (int64_t)pool;
+  // A threshold pass pays where its sample can hold the pool, but not for a query or two of a few
+  // hundred references, whose insertions take less than its two launches (whole calls, us,
+  // without / with: one query, pool 64, 700 references 51 / 58, 1024 64 / 57; pool 20, 1500
+  // 55 / 61, 2000 63 / 59; FP32, 512 136 / 125; two of 500, pool 64, 54 / 58; ten 127 / 58).
+  p.bounded = nr >= 8 * (int64_t)pool &&
+              (double)nq * (double)nr * std::sqrt((double)pool) * (dtype == SH_F32 ? 4 : 1) >= 8000.0;
   // Measured time of a pair in the scan's loop: 0.1 ps for 64 packed BF16 elements, FP8 half,
   // FP32 0.75 ps for 56.
   const double c_pair = dtype == SH_F32    ? 0.75e-12 * K / 56

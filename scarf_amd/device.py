@@ -4,7 +4,6 @@ and to name the current HIP stream.
 """
 from __future__ import annotations
 
-import contextlib
 import ctypes
 import dataclasses
 import threading
@@ -36,20 +35,17 @@ def stream_handle(stream=None) -> ctypes.c_void_p:
 
 
 class Workspace:
-    """A growable byte buffer reused across calls on one stream."""
+    """A growable byte buffer reused across calls on one stream.
+
+    ``lock`` is held from ``get`` to the end of a library call whose kernels hand results on
+    in the buffer.  A call gives the interpreter away while it queues them, so another thread
+    with the same stream could queue its own in between; the stream keeps the order only of
+    whole calls."""
 
     def __init__(self, device="cuda"):
         self.device = device
         self.buf = None
         self.lock = threading.Lock()
-
-    @contextlib.contextmanager
-    def hold(self, nbytes: int):
-        """The buffer for one library call whose kernels hand results on in it.  A call gives
-        the interpreter away while it queues them, so another thread with the same stream
-        could queue its own in between; the stream keeps the order only of whole calls."""
-        with self.lock:
-            yield self.get(nbytes)
 
     def get(self, nbytes: int):
         nbytes = max(int(nbytes), 256)

@@ -130,7 +130,9 @@ def locality_order(E: "torch.Tensor", stream=None) -> "torch.Tensor":
     perm = torch.empty(n, dtype=torch.int64, device=E.device)
     if n == 0:
         return perm
-    with workspace("order").hold(_lib.lib().sh_locality_order_workspace(n)) as (buf, nbytes):
+    ws = workspace("order")
+    with ws.lock:
+        buf, nbytes = ws.get(_lib.lib().sh_locality_order_workspace(n))
         _lib.call("sh_locality_order", ptr(E), n, D, E.stride(0), ptr(perm), ptr(buf), nbytes,
                   stream_handle(stream))
     return perm
@@ -267,20 +269,20 @@ def _search(Q, R, refs, k, pool, self_offset, n_slices, certify, self_idx, strea
             seeds = None
         cand = torch.empty((nq, S, pool), dtype=torch.int64, device=dev)
         cnt = torch.empty((nq, S), dtype=torch.int32, device=dev)
-        need = _lib.lib().sh_knn_screen_workspace(nq, pool, S)
-        with workspace("screen").hold(need) as (ws, nbytes), \
-                kernel_timer("screen", stream, flops=2.0 * nq * nr * D):
+        ws = workspace("screen")
+        with ws.lock, kernel_timer("screen", stream, flops=2.0 * nq * nr * D):
+            buf, nbytes = ws.get(_lib.lib().sh_knn_screen_workspace(nq, pool, S))
             _lib.call("sh_knn_screen", ptr(qp), nq, ptr(refs.data), nr, D, code, None, None,
-                      pool, S, ptr(seeds), ptr(cand), ptr(cnt), ptr(ws), nbytes, st)
+                      pool, S, ptr(seeds), ptr(cand), ptr(cnt), ptr(buf), nbytes, st)
     else:
         S = 1
         cand = torch.empty((nq, pool), dtype=torch.int64, device=dev)
         cnt = torch.empty(nq, dtype=torch.int32, device=dev)
-        need = _lib.lib().sh_knn_pool_workspace(nq, nr, D, code, pool)
-        with workspace("screen").hold(need) as (ws, nbytes), \
-                kernel_timer("screen", stream, flops=2.0 * nq * nr * D):
+        ws = workspace("screen")
+        with ws.lock, kernel_timer("screen", stream, flops=2.0 * nq * nr * D):
+            buf, nbytes = ws.get(_lib.lib().sh_knn_pool_workspace(nq, nr, D, code, pool))
             _lib.call("sh_knn_pool", ptr(qp), nq, ptr(refs.data), nr, D, code, pool, ptr(cand),
-                      ptr(cnt), ptr(ws), nbytes, st)
+                      ptr(cnt), ptr(buf), nbytes, st)
     if certify is None:
         certify = refs.dtype in ("fp32", "f32")
     err_coef = -1.0
