@@ -9,7 +9,10 @@ Scheduling
 ----------
 * Admission by memory: a request is admitted when its device footprint (counts,
   neighbour tables, score vector) fits in what is left of ``mem_budget``; requests
-  that could never fit are rejected with an error.  Admission is FIFO.
+  that could never fit are rejected with an error.  Admission is FIFO.  The budget holds
+  requests only: each stream also keeps the workspace of its searches, which
+  ``search_bytes`` bounds (8.1 GB for four streams, chunks of 16,384 cells and a BF16
+  index of 500,000).
 * Requests are split into chunks of at most ``chunk_rows`` cells.  The engine issues
   chunks round-robin over the admitted requests, each on one of ``n_streams`` HIP
   streams, so a small request that arrives while a large one is on the GPU is admitted
@@ -41,7 +44,7 @@ import numpy as np
 
 from . import _lib
 from .device import DeviceCSR, col_map_from_positions, ptr, require_gpu, stream_handle, workspace
-from .knn import GpuIndex, search
+from .knn import REFINE_POOL, GpuIndex, search
 from .mapping import align_col_map
 from .normalize import NormParams
 from .pca import Projector
@@ -131,6 +134,21 @@ class MappingServer:
         n = csr.n_rows
         return (csr.nnz * 8 + (n + 1) * 8 + n * self.k * 12
                 + self.n_ref * 16 + 4096)
+
+    @property
+    def search_bytes(self) -> int:
+        """Device bytes that the streams' search workspaces can come to, beside
+        ``mem_budget``: the largest need of a chunk of up to ``chunk_rows`` cells on every
+        stream, with the quarter that a workspace grows by."""
+        L, code = _lib.lib(), _lib.DTYPES[self.refs.dtype]
+        pools = [max(self.index.pool, self.k)]
+        if self.refs.dtype == "fp8" and pools[0] < REFINE_POOL:
+            pools.append(REFINE_POOL)
+        # the need is linear in the queries of a 256-query block
+        sizes = list(range(256, self.chunk_rows, 256)) + [self.chunk_rows]
+        need = max(L.sh_knn_pool_workspace(n, self.n_ref, self.refs.D, code, p)
+                   for p in pools for n in sizes)
+        return len(self.streams) * (max(need, 256) * 5 // 4 + 256)
 
     def submit(self, csr, arrival: Optional[float] = None) -> cf.Future:
         if csr.n_cols != self.n_cols:

@@ -145,3 +145,27 @@ def test_cancel_frees_slot_and_memory(server_setup):
     np.testing.assert_array_equal(after.indices, alone.indices)
     np.testing.assert_array_equal(after.distances, alone.distances)
     np.testing.assert_array_equal(after.scores, alone.scores)
+
+
+@pytest.mark.parametrize("screen", ["bf16", "fp8"])
+def test_search_bytes_bounds_the_streams_workspaces(server_setup, screen):
+    """What the streams' searches hold beside the admission budget, after chunks of several
+    sizes, is within what the server says."""
+    from scarf_amd import device
+    from scarf_amd.knn import GpuIndex
+    ann, src_ids, q_ids, pool = server_setup
+    say("serving search bytes", screen)
+    E = ann.annIdx.embedding()
+    index = GpuIndex("l2", E.shape[1], screen=screen, pool=64 if screen == "bf16" else 128)
+    index.init_index(E.shape[0])
+    index.add_items(E)
+    from scarf_amd.serving import MappingServer
+    with MappingServer(ann.loadings, ann.mu, ann.sigma, index, src_ids, q_ids, norm=ann.data.norm,
+                       k=11, chunk_rows=2000, n_streams=3) as srv:
+        keys = [("screen", s.cuda_stream) for s in srv.streams]
+        for key in keys:  # a stream of the pool may have served another test
+            device._workspaces.pop(key, None)
+        for n in (1, 300, 1999, 2001, 4400):
+            assert srv.submit(_req(pool, 0, n)).result(timeout=60).error is None
+        held = [device._workspaces[key].buf.numel() for key in keys if key in device._workspaces]
+        assert held and sum(held) <= srv.search_bytes
