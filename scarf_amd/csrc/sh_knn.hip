@@ -322,7 +322,7 @@ __global__ void __launch_bounds__(256) k_pool_merge(
       for (; bit >= 0 && !cut; --bit) {
         const uint32_t t = prefix | ((1u << bit) - 1u);
         int c = 0;
-        if constexpr (BITS) {  // a large scan: many waves, and groups past m are skipped
+        if constexpr (BITS) {  // k_collect's keys: many waves, and groups past m are skipped
 #pragma unroll
           for (int i = 0; i < E; ++i)
             if (64 * i < m)
@@ -977,8 +977,7 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
   // 55 / 61, 2000 63 / 59; FP32, 512 136 / 125; two of 500, pool 64, 54 / 58; ten 127 / 58).
   p.bounded = nr >= 8 * (int64_t)pool &&
               (double)nq * (double)nr * std::sqrt((double)pool) * (dtype == SH_F32 ? 4 : 1) >= 8000.0;
-  // Measured time of a pair in the scan's loop: 0.1 ps for 64 packed BF16 elements, FP8 half,
-  // FP32 0.75 ps for 56.
+  // Measured time of a pair in the scan's loop.
   const double c_pair = dtype == SH_F32    ? 0.75e-12 * K / 56
                         : dtype == SH_BF16 ? 0.1e-12 * K / 64
                                            : 0.055e-12 * K / 64;
@@ -992,12 +991,12 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
   p.len3 = align_up((size_t)nr, kSliceAlign);
   if (p.bounded) {
     // A sample of 1 / s of the rows costs nr * c_pair / s per query and leaves rank * s keys
-    // (a tenth more for minima that share a slot) to insert.  Measured: c_pair 0.1 ps per
-    // pair of 64 packed BF16 elements (FP8 half, FP32 0.75 ps per 56); a key costs 37 ps
-    // where a tile of 32 references x 64 queries meets three of them and 80 ps where it
-    // meets one in two tiles (the tile leaves the short path for it alone), twice that for
-    // FP8.  The million-cell self search takes 174 / 152 / 146 / 146 ms with s = 2 / 4 / 8 /
-    // 16, the 100,000-cell one 2.91 / 2.68 / 2.67 / 2.87.
+    // (a tenth more for minima that share a slot) to insert.  Measured: a key costs 37 ps where a
+    // tile of 32 references x 64 queries meets three of them and 80 ps where it meets one in two
+    // tiles (the tile leaves the short path for it alone), twice that for FP8.  Self searches with
+    // s = 1 / 2 / 4 / 8 / 16: a million cells 216 / 172 / 149 / 143 / 142 ms (16 is taken), 100,000
+    // 2.92 / 2.64 / 2.43 / 2.41 / 2.55 (4), 19,001 in FP32 1.02 / 0.88 / 0.79 / 0.76 / 0.76 (8),
+    // 300,000 in FP8 24.6 / 23.2 / 23.9 / 23.6 / 24.1 (4).
     double best = 0.0;
     for (int sh = 0; sh <= 4; ++sh) {
       if (sh > 0 && (nr >> sh) < 8 * (int64_t)pool) break;
@@ -1013,7 +1012,7 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
       }
     }
     p.m = nr >> p.shift;
-    const int64_t res1 = (int64_t)ops.bound_resident(K) * kCUs;
+    const int64_t res1 = (int64_t)ops.scan_resident(K) * kCUs;
     // at most 256 slices here and 512 below: one query's slots and segments are one wave's
     // work, and past that it takes longer than the slices save
     const int max1 = (int)std::min<int64_t>(256, cdiv(p.m, kSliceAlign));
@@ -1030,7 +1029,7 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
     p.slots = p.S1 * 2 * p.per;
     int64_t res3;
     if (p.collect) {
-      res3 = (int64_t)ops.collect_resident(K) * kCUs;
+      res3 = (int64_t)ops.scan_resident(K) * kCUs;
       // a query's keys vary with the sample by 1 / sqrt(rank); all may come from one slice
       const double keys = 1.1 * p.rank * (1 << p.shift);
       p.cap = (int)align_up((size_t)(keys * (1.0 + 7.5 / std::sqrt((double)p.rank))) + 64, 128);
@@ -1054,7 +1053,7 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
   p.batch3 = nq;
   if (p.collect) {  // whole fills of the GPU a launch
     const int64_t most = (int64_t)(kBufBytes / ((size_t)p.S3 * p.cap * 8));
-    const int64_t fill = (int64_t)ops.collect_resident(K) * kCUs * 256;
+    const int64_t fill = (int64_t)ops.scan_resident(K) * kCUs * 256;
     p.batch3 = std::min(nq, most >= fill ? most / fill * fill
                                          : std::max<int64_t>(256, most / 256 * 256));
   }
@@ -1084,7 +1083,7 @@ static PoolPlan pool_plan(int64_t nq, int64_t nr, int K, int dtype, int pool) {
 static bool pool_built(int dtype, int32_t D) {
   const KnnOps ops = knn_ops(dtype);
   const int32_t K = pack_k(dtype, D);
-  return ops.bound && K > 0 && ops.bound_resident(K) > 0 && ops.collect_resident(K) > 0;
+  return ops.bound && K > 0 && ops.scan_resident(K) > 0;
 }
 
 struct MergeArgs {

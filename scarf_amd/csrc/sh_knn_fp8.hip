@@ -5,8 +5,8 @@ namespace sh {
 
 using Table = KnnTable<OpFP8, true, 64, 128>;
 KnnOps knn_ops_fp8() {
-  return {Table::screen,          Table::bound,          Table::collect,
-          Table::screen_resident, Table::bound_resident, Table::collect_resident};
+  return {Table::screen, Table::bound, Table::collect, Table::screen_resident,
+          Table::scan_resident};
 }
 
 }  // namespace sh

@@ -557,14 +557,15 @@ __device__ __forceinline__ int64_t sample_row(int64_t i, int shift) {
   return (i << shift) + (int64_t)((x >> 16) & ((1u << shift) - 1u));
 }
 
+// Resident workgroups per CU of k_bound and k_collect.
 template <class Op, int K>
-constexpr int bound_minb() {
+constexpr int scan_minb() {
   if constexpr (Op::kScaled) return K >= 128 ? 3 : 4;
   return K * Op::ESZ <= 128 ? 4 : K * Op::ESZ <= 256 ? 3 : 2;
 }
 
 template <class Op, int K>
-__global__ void __launch_bounds__(256, (bound_minb<Op, K>())) k_bound(
+__global__ void __launch_bounds__(256, (scan_minb<Op, K>())) k_bound(
     const typename Op::Frag *__restrict__ Qp_, int64_t nq, const unsigned char *__restrict__ Rp,
     int64_t m, int shift, int64_t slice_len, int S, int per, float *__restrict__ slot_min) {
   typedef typename Op::Frag Frag;
@@ -710,7 +711,8 @@ __global__ void __launch_bounds__(256, (bound_minb<Op, K>())) k_bound(
 }
 
 // ---------------------------------------------------------------------------------
-// The scan of a large search: k_screen's tile loop against a threshold that does not move.
+// The scan of all but the smallest searches (pool_plan): k_screen's tile loop against a threshold
+// that does not move.
 //
 // With a threshold per query from k_bound the scan meets a few hundred keys per query, so
 // it needs no compaction, no sort and no seeds: a passing key goes to the lane half's
@@ -726,13 +728,7 @@ __global__ void __launch_bounds__(256, (bound_minb<Op, K>())) k_bound(
 // 20.2 ms: the matrix cores at the clock that this load leaves them.  Four query groups per
 // wave at two workgroups per CU: 25.7 and 32.6 ms, so the smaller block was kept.
 template <class Op, int K>
-constexpr int collect_minb() {
-  if constexpr (Op::kScaled) return K >= 128 ? 3 : 4;
-  return K * Op::ESZ <= 128 ? 4 : K * Op::ESZ <= 256 ? 3 : 2;
-}
-
-template <class Op, int K>
-__global__ void __launch_bounds__(256, (collect_minb<Op, K>())) k_collect(
+__global__ void __launch_bounds__(256, (scan_minb<Op, K>())) k_collect(
     const typename Op::Frag *__restrict__ Qp_, int64_t nq, const unsigned char *__restrict__ Rp,
     int64_t nr, int64_t slice_len, int S, const float *__restrict__ tau0, int cap,
     uint2 *__restrict__ buf, int32_t *__restrict__ seg_cnt) {
@@ -955,8 +951,7 @@ struct KnnOps {  // false / 0: no such instantiation
   bool (*bound)(int K, const BoundArgs &, hipStream_t);
   bool (*collect)(int K, const CollectArgs &, hipStream_t);
   int (*screen_resident)(int K, int cap);  // workgroups per CU
-  int (*bound_resident)(int K);
-  int (*collect_resident)(int K);
+  int (*scan_resident)(int K);
 };
 KnnOps knn_ops_bf16();
 KnnOps knn_ops_fp8();
@@ -1015,11 +1010,6 @@ struct KnnTable {
     ((K == KS ? (launch_collect<Op, KS>(a, st), (void)(ok = true)) : (void)0), ...);
     return ok;
   }
-  static int collect_resident(int K) {
-    int n = 0;
-    ((K == KS ? (void)(n = collect_minb<Op, KS>()) : (void)0), ...);
-    return n;
-  }
   static int screen_resident(int K, int cap) {
     int n = 0;
     ((K == KS ? (void)(n = cap == 256 ? screen_minb<Op, KS, 256>()
@@ -1029,9 +1019,9 @@ struct KnnTable {
      ...);
     return n;
   }
-  static int bound_resident(int K) {
+  static int scan_resident(int K) {
     int n = 0;
-    ((K == KS ? (void)(n = bound_minb<Op, KS>()) : (void)0), ...);
+    ((K == KS ? (void)(n = scan_minb<Op, KS>()) : (void)0), ...);
     return n;
   }
 };

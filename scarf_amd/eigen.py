@@ -587,20 +587,3 @@ class _DeviceBlock:
         scale = max(abs(theta[order[0]]), np.finfo(float).tiny)
         orth = float(np.max(np.abs(HG[1] - np.eye(n))))
         return theta[order], Vh[order], float(np.max(res)) / scale, orth
-
-
-def _verify_rows(M, Vt, d, st):
-    """Rayleigh quotients of the rows of Vt (device, n x d) under M, sorted descending,
-    with the largest relative residual and the orthogonality defect (one FP64 GEMM)."""
-    n_top = int(Vt.shape[0])
-    Y = torch.empty((n_top, d), dtype=torch.float64, device=M.device)
-    _lib.call("sh_dgemm", 0, n_top, d, d, 1.0, ptr(Vt), d, ptr(M), d, 0.0, ptr(Y), d, st)
-    Vh = Vt.cpu().numpy()
-    Yh = Y.cpu().numpy()
-    theta = np.einsum("ij,ij->i", Yh, Vh)
-    order = np.argsort(-theta, kind="stable")
-    theta, Vh, Yh = theta[order], Vh[order], Yh[order]
-    scale = max(abs(theta[0]), np.finfo(float).tiny)
-    res = float(np.max(np.linalg.norm(Yh - theta[:, None] * Vh, axis=1))) / scale
-    orth = float(np.max(np.abs(Vh @ Vh.T - np.eye(n_top))))
-    return theta, Vh, res, orth

@@ -225,7 +225,7 @@ def _search_ordered(Q, R, refs, k, pool, self_offset, n_slices, certify, self_id
         si_s = permute_rows(si, perm, stream=stream).view(-1)
     elif self_offset is not None:
         si_s = perm + int(self_offset)
-        if seed:  # distinct rows of R, near each other in locality order
+        if seed and n_slices:  # distinct rows of R, near each other in locality order
             seeds = si_s
     else:
         si_s = None
