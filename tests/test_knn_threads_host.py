@@ -2,6 +2,7 @@
 several kernels that hand results on in a workspace, and the stream's workspace is one: another
 thread's call on the same buffer must not come between them."""
 import functools
+import os
 import threading
 import time
 import types
@@ -10,6 +11,9 @@ import pytest
 import torch
 
 from scarf_amd import _lib, device, knn
+
+pytestmark = pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH),
+                                reason="libscarfhip.so not built")
 
 
 @pytest.fixture
